@@ -73,7 +73,7 @@ DOWN_BYTES = HIDDEN * BLOCKS * 17         # 4,406,400 B per expert
 SEED = 20251201
 RMS_EPS = 1e-5  # GPT-OSS rms_norm_eps
 COPY_PROBE_BYTES = 1 << 30  # device copy that calibrates the HBM byte counters
-GATE_UP_KERNEL = re.compile(r"gemm_kernel<.*>, 1, (true|false)>|gemv_kernel<1, \d+, \d+>|route_gemv_kernel")
+GATE_UP_KERNEL = re.compile(r"gemm_kernel<.*>, 1, (true|false)>|gemm_wide_kernel<1, (true|false)>|gemv_kernel<1, \d+, \d+>|route_gemv_kernel")
 
 CONFIGS = {
     0: {"batch": 1, "layers": 12, "experts": 32, "routing": "router", "zipf": None, "roofline": "hbm",

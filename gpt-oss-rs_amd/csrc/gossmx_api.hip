@@ -826,13 +826,22 @@ void gossmx_weights_destroy(gossmx_weights* w) {
   delete w;
 }
 
-// Rows per GEMM work item for a batch of m activation rows (it selects the
-// kernel geometry). Batches of at most kSmallChunk rows: every bucket is one
-// work item (more work-groups, fewer sequential K steps). Batches of at least
-// kHugeMinRows rows: 32-row items share each weight block's conversion.
-static int gemm_chunk(size_t m) {
+// Rows per GEMM work item for a batch of m activation rows and `routes` (row,
+// expert) pairs over `experts` (it selects the kernel geometry). Batches of at
+// most kSmallChunk rows: every bucket is one work item (more work-groups,
+// fewer sequential K steps). 32-row items on the scaled MFMA from
+// kWideRoutes routes and kWideRows rows per expert on: below, a 32-row item
+// holds mostly padding, or its 256-row work-groups leave CUs idle (20B shape,
+// residual-Q8, 16- against 32-row items: 128 rows 178 against 187 us, 256 rows
+// 268 / 272, 352 rows 333 / 319, 500 rows 448 / 399; 128 experts, 512 rows 684
+// / 655). Q8 items, with half the chain, and the full items of a single
+// expert gain earlier (Q8 128 rows 169 / 147; one 5,760-row expert, 400 rows 56
+// / 61, 512 rows 69 / 64).
+constexpr size_t kWideRows = 16, kWideRoutes = 1280, kWideRoutesQ8 = 512;
+static int gemm_chunk(size_t m, size_t routes, size_t experts, bool residual) {
   if (m <= (size_t)kSmallChunk) return kSmallChunk;
-  return m >= (size_t)kHugeMinRows ? kHugeChunk : kChunk;
+  const size_t least = residual && experts > 1 ? kWideRoutes : kWideRoutesQ8;
+  return routes >= std::max(least, kWideRows * experts) ? kHugeChunk : kChunk;
 }
 
 // Batches of at most kTinyMaxRows rows on weights of at most kTinyMaxBlocks
@@ -870,7 +879,10 @@ static int matmul_impl(gossmx_ctx* ctx, const gossmx_matmul_problem* p) {
   }
   if (int s = ensure(ctx, ctx->act1v, m * B * 2 * kBlock * sizeof(_Float16) + kActSlack)) return s;
   if (int s = ensure(ctx, ctx->act1s, m * B * 2 * sizeof(float) + kActSlack)) return s;
-  ActBuffers act{static_cast<_Float16*>(ctx->act1v.p), static_cast<float*>(ctx->act1s.p)};
+  const bool gemv = use_gemv(m, B, p->activation_kind == GOSSMX_ACT_RESIDUAL_Q8);
+  const int chunk = gemm_chunk(m, m, 1, p->activation_kind == GOSSMX_ACT_RESIDUAL_Q8);
+  ActBuffers act{static_cast<_Float16*>(ctx->act1v.p), static_cast<float*>(ctx->act1s.p),
+                 !gemv && chunk == kHugeChunk ? 1 : 0};
   HIP_TRY(launch_prep_records(rec, p->activation_kind, m, B, p->row_stride, act, ctx->err, ctx->stream),
           "prepare activations");
   const float* bias = p->bias;
@@ -902,14 +914,12 @@ static int matmul_impl(gossmx_ctx* ctx, const gossmx_matmul_problem* p) {
   g.bias_expert_stride = 0;  // this problem's single bias vector
   begin_call(ctx, m, m, p->memory, context_scratch_bytes(ctx));
   {
-    const bool gemv = use_gemv(m, B, g.residual != 0);
     KernelScope scope(ctx, GOSSMX_OP_MATMUL,
                       {GOSSMX_ROLE_NONE, gemv ? GOSSMX_KERNEL_GEMV : GOSSMX_KERNEL_GEMM, (uint32_t)rows,
-                       (uint32_t)(B * kBlock), gemv ? 0u : (uint32_t)gemm_chunk(m)});
+                       (uint32_t)(B * kBlock), gemv ? 0u : (uint32_t)chunk});
     if (gemv) {
       HIP_TRY(launch_gemv(kPlain, g, (int)m, 1, ctx->stream, scope.start, scope.stop), "matmul launch");
     } else {
-      const int chunk = gemm_chunk(m);
       HIP_TRY(launch_gemm(kPlain, g, chunk, (int)((m + chunk - 1) / chunk), ctx->stream, scope.start, scope.stop),
               "matmul launch");
     }
@@ -1029,7 +1039,7 @@ static int moe_forward_impl(gossmx_ctx* ctx, const gossmx_layer* L, const gossmx
   if (int s = set_device(ctx->device)) return s;
   const bool host = io->memory == GOSSMX_MEM_HOST;
   const int proj = L->cfg.projection;
-  const int chunk = gemm_chunk(m);
+  const int chunk = gemm_chunk(m, R, E, proj == GOSSMX_PROJECTION_RESIDUAL_Q8);
   const size_t max_work = (R + chunk - 1) / chunk + std::min(E, R);
 
   // Scratch: the context's grow-only buffers, or the no-allocation entry
@@ -1052,6 +1062,7 @@ static int moe_forward_impl(gossmx_ctx* ctx, const gossmx_layer* L, const gossmx
       (s = take(ctx, arena, ctx->act2s, R * B2 * 8 + kActSlack, &act2.s)) ||
       (s = take(ctx, arena, ctx->y, R * H * 2, &ybuf)))
     return s;
+  act1.digits = act2.digits = proj != GOSSMX_PROJECTION_EXACT_BF16 && chunk == kHugeChunk ? 1 : 0;
   // Batches whose logits fit one work-group take the fused selection +
   // dispatch kernel; larger ones a selection kernel with per-work-group
   // expert counts and a placement kernel. The router projection (when the

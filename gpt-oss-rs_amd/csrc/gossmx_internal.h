@@ -14,8 +14,7 @@ constexpr int kTileRows = 16;   // rows per MFMA tile (one wave)
 constexpr int kWgRows = 64;     // gate_up rows (32 gate/up pairs) per 32-value block of the down input
 constexpr int kChunk = 16;      // activation rows per GEMM work item (batches of more than kSmallChunk rows)
 constexpr int kSmallChunk = 8;  // activation rows per work item for batches of at most 8 rows
-constexpr int kHugeChunk = 32;  // activation rows per work item for batches of at least kHugeMinRows rows
-constexpr int kHugeMinRows = 512;
+constexpr int kHugeChunk = 32;  // activation rows per work item where experts hold many rows (gemm_chunk)
 constexpr int kChunkMax = 32;
 // Small-batch GEMV (gemv_kernel): batches of at most kTinyMaxRows rows whose
 // blocks per row are at most kTinyMaxBlocks (the activation image of the
@@ -48,10 +47,12 @@ struct TiledWeights {
   size_t experts = 0, rows = 0, blocks = 0, tiles = 0;
   size_t nib_stride = 0;  // bytes per expert in the nibble plane
   size_t scl_stride = 0;  // bytes per expert in the scale plane
-  // [experts][tiles]: 1 when every scale byte of the tile is in the exact
-  // scaled-conversion range (see tile_flags_kernel); set after every write.
+  // [experts][tiles]: kTileFast when every scale byte of the tile is in the
+  // exact scaled-conversion range, kTileWide when every one is in the scaled
+  // MFMA's (see tile_flags_kernel); set after every write.
   uint8_t* fast = nullptr;
 };
+constexpr int kTileFast = 1, kTileWide = 2;
 
 // Extra bytes allocated after each plane: the GEMM reads whole 4-block groups
 // (and dword-granular tails) of the last tile unconditionally.
@@ -64,9 +65,15 @@ constexpr size_t kActSlack = 2048;
 // Activation operand of the expert GEMM, one row per token or route:
 //  actv [row][block][part 0 = primary, 1 = residual][32] f16 (the Q8 codes,
 //  exact in f16), acts [row][block][2] f32 (primary scale, residual scale).
+// With `digits` (the operand of gemm_wide_kernel) v holds [row][block] records
+// of kDigitRecord bytes instead: per part 48 bytes, the code's low and high
+// digit as 32 six-bit values (24 bytes) each, stored as low bytes 0-15, high
+// bytes 0-15, low bytes 16-23, high bytes 16-23.
+constexpr int kDigitRecord = 96;
 struct ActBuffers {
   _Float16* v = nullptr;
   float* s = nullptr;
+  int digits = 0;
 };
 
 enum GemmMode { kPlain = 0, kGateUp = 1, kDown = 2 };

@@ -169,6 +169,11 @@ __device__ __forceinline__ float half_wave_max(float m) {
   return fmaxf(m, __uint_as_float(lane_partner<16>(__float_as_uint(m))));
 }
 
+// roundf (half away from zero) of |x| < 2^23: adding the float below 0.5 with
+// x's sign and truncating gives roundf's bits (compared on every such float),
+// in three instructions.
+__device__ __forceinline__ float round_half_away(float x) { return truncf(x + copysignf(0x1.fffffep-2f, x)); }
+
 // quantize_q8_block (lib.rs:1051-1065) for the 32 values held by a 32-lane
 // half wave (lane l32 holds value l32): scale = max|v| / 127, inverse =
 // 1 / scale (0 when scale is 0), q = clamp(round_half_away(v * inverse)).
@@ -180,8 +185,32 @@ __device__ __forceinline__ void q8_half_wave(float v, float& q, float& scale) {
   q = fminf(fmaxf(roundf(v * inv), -127.0f), 127.0f);
 }
 
+// One Q8 code's two sign-magnitude digits (q = 16 high + low, both carrying
+// q's sign) as six-bit E2M3 codes packed into a part's 48-byte record (see
+// ActBuffers): code sign << 5 | d is d / 8 for every digit d <= 15. The half
+// wave's lane l32 holds value l32; four lanes' codes make three bytes, which
+// lanes 0..2 of the quad store. Every lane of the half wave calls it.
+__device__ __forceinline__ uint32_t quad_or(uint32_t v) {
+  v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, false);
+  return v;
+}
+__device__ __forceinline__ void store_digits(uint8_t* rec, float qf, int l32, bool store = true) {
+  const int q = (int)qf;
+  const uint32_t sign = q < 0 ? 32u : 0u, mag = (uint32_t)(q < 0 ? -q : q);
+  const int k = l32 & 3;
+  const uint32_t lo = quad_or((sign | (mag & 15u)) << (6 * k)), hi = quad_or((sign | (mag >> 4)) << (6 * k));
+  const int b = 3 * (l32 >> 2) + k;  // byte of the digit's 24
+  if (store && k < 3) {
+    uint8_t* p = rec + (b < 16 ? b : b + 16);
+    p[0] = (uint8_t)(lo >> (8 * k));
+    p[b < 16 ? 16 : 8] = (uint8_t)(hi >> (8 * k));
+  }
+}
+
 // quantize_residual_q8 (lib.rs:382-409) of one block held by a half wave;
-// writes the f16 codes and the two scales of (row, blk) into `act`. With
+// writes the codes (f16, or with act.digits the digit records) and the two
+// scales of (row, blk) into `act`. With
 // qmode kProjQ8, quantize_q8 (lib.rs:347-378): the primary block only, the
 // residual codes and scale stored as zeros. With kProjExactBf16 the value's
 // bf16 bits go to act.v viewed as [row][blocks * 32] bf16.
@@ -196,9 +225,15 @@ __device__ __forceinline__ void residual_q8_store(float v, int l32, size_t row, 
   const float r = qmode == kProjQ8 ? 0.0f : v - q * s;
   float rq, rs;
   q8_half_wave(r, rq, rs);
-  _Float16* dst = act.v + ((row * blocks + blk) * 2) * kBlock;
-  dst[l32] = (_Float16)q;
-  dst[kBlock + l32] = (_Float16)rq;
+  if (act.digits) {
+    uint8_t* rec = reinterpret_cast<uint8_t*>(act.v) + (row * blocks + blk) * kDigitRecord;
+    store_digits(rec, q, l32);
+    store_digits(rec + kDigitRecord / 2, rq, l32);
+  } else {
+    _Float16* dst = act.v + ((row * blocks + blk) * 2) * kBlock;
+    dst[l32] = (_Float16)q;
+    dst[kBlock + l32] = (_Float16)rq;
+  }
   if (l32 == 0) {
     float2 sc;
     sc.x = s;
@@ -231,7 +266,7 @@ __device__ __forceinline__ void q8_scales_n(const float (&mx)[N], int l32, float
 // hw + i * stride: activation row first_row + item / per_row, block
 // first_blk + item % per_row); blocks with live[i] false are computed on
 // zeros and not stored. The same operations as residual_q8_store per block.
-template <int N, bool RESIDUAL>
+template <int N, bool RESIDUAL, bool DIGITS = false>
 __device__ __forceinline__ void residual_q8_store_n(const float (&v)[N], const bool (&live)[N], int l32, int hw,
                                                     int stride, int per_row, size_t first_row, int blocks,
                                                     int first_blk, ActBuffers act) {
@@ -272,9 +307,15 @@ __device__ __forceinline__ void residual_q8_store_n(const float (&v)[N], const b
     const int item = hw + i * stride;
     const size_t row = first_row + item / per_row;
     const int blk = first_blk + item % per_row;
-    _Float16* dst = act.v + ((row * blocks + blk) * 2) * kBlock;
-    dst[l32] = (_Float16)q[i];
-    dst[kBlock + l32] = (_Float16)rq[i];
+    if (DIGITS) {
+      uint8_t* rec = reinterpret_cast<uint8_t*>(act.v) + (row * blocks + blk) * kDigitRecord;
+      store_digits(rec, q[i], l32);
+      if (RESIDUAL) store_digits(rec + kDigitRecord / 2, rq[i], l32);
+    } else {
+      _Float16* dst = act.v + ((row * blocks + blk) * 2) * kBlock;
+      dst[l32] = (_Float16)q[i];
+      dst[kBlock + l32] = (_Float16)rq[i];
+    }
     if (l32 == 0) {
       float2 sc;
       sc.x = s[i];
@@ -1200,21 +1241,8 @@ typedef __attribute__((address_space(3))) void* lds_ptr;
 //    rows, whose work items are one expert each and whose time is the weight
 //    stream's latency: 64-row work-groups (four times the big geometry's
 //    count per expert), 73 VGPRs, 5 work-groups per CU.
-//  GemmHuge (2 tiles, 32 rows, 4 blocks, 8 waves) serves prefill-sized
-//    batches, where the FP4->f16 conversion of a weight block is shared by
-//    four token groups. Its gate_up grid pins weight tiles to XCDs (PIN_XCD).
-//
-// PIN_XCD: work-groups reach the eight XCDs round-robin in launch order, so
-// with a grid row of n_x work-groups the chunks of one expert (consecutive
-// rows) would read the same tile through different L2s whenever n_x is not a
-// multiple of 8. A pinned gate_up grid pads its rows to a multiple of 8
-// (padding work-groups return at once) and rotates each row by the item's
-// expert, so tile column x of expert e always runs on XCD (x + e) mod 8: the
-// later chunks of a popular expert hit the L2 the first one filled, and the
-// XCDs that get one column fewer differ from expert to expert. It pays when
-// experts have many chunks (prefill); with one or two chunks per expert the
-// padding's imbalance costs more than the L2 hits save.
-template <int TILES, int NTOK, int GROUPS, int WAVES = 8, int MIN_WAVES = 4, int WLEAD = 2, bool PIN_XCD = false>
+// Batches whose experts hold many rows run gemm_wide_kernel instead.
+template <int TILES, int NTOK, int GROUPS, int WAVES = 8, int MIN_WAVES = 4, int WLEAD = 2>
 struct GemmCfg {
   static constexpr int kWaves = WAVES;                    // waves per work-group
   static constexpr int kThreads = 64 * WAVES;
@@ -1236,7 +1264,6 @@ struct GemmCfg {
   // Steps by which the weight requests lead their use (1 or 2; the DMA leads
   // by 2).
   static constexpr int kWLead = WLEAD;
-  static constexpr bool kPinXcd = PIN_XCD;  // gate_up grid rows pinned to XCDs (above)
   // s_waitcnt immediate for "the DMA and the weights of step q have landed":
   // issued after them are D(q+1) and, with a two-step lead, W(q+1) (see
   // k_loop). expcnt and lgkmcnt are not waited on.
@@ -1252,9 +1279,7 @@ struct GemmCfg {
 };
 using GemmBig = GemmCfg<2, 16, 1, 4, 5>;
 using GemmSmall = GemmCfg<1, 8, 2, 4, 5>;
-using GemmHuge = GemmCfg<2, 32, 1, 8, 4, 1, true>;
-static_assert(GemmBig::kChunk == kChunk && GemmSmall::kChunk == kSmallChunk && GemmHuge::kChunk == kHugeChunk,
-              "work item sizes");
+static_assert(GemmBig::kChunk == kChunk && GemmSmall::kChunk == kSmallChunk, "work item sizes");
 constexpr int kBufferFlags = 0x00020000;    // raw 32-bit buffer resource, gfx9 family
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base) {
@@ -1471,8 +1496,8 @@ __device__ __forceinline__ void step_pipelined(Acc<C>& tot, const char* codes, c
 template <class C, int MODE, bool RESIDUAL, bool TABLE = false>
 __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, const Acc<C>& tot, const int n_tg, const int count,
                                               const int start, const int tile0, float* s_act,
-                                              const int* s_slot = nullptr, int wg_x = -1) {
-  if (wg_x < 0) wg_x = (int)blockIdx.x;  // the work-group's tile column
+                                              const int* s_slot = nullptr) {
+  const int wg_x = (int)blockIdx.x;  // the work-group's tile column
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int nl = lane & 15, G = lane >> 4;
@@ -1735,14 +1760,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void gemm_kernel(GemmArg
     count = rec.z;
   }
   const int rows = (int)a.w.rows, B = (int)a.w.blocks;
-  int wg_x = (int)blockIdx.x;  // tile column
-  if (C::kPinXcd && MODE == kGateUp) {
-    const int n_x = ((int)a.w.tiles + C::kWgTiles - 1) / C::kWgTiles;
-    const int p_x = (int)gridDim.x;  // n_x padded to a multiple of 8
-    wg_x = ((int)blockIdx.x + p_x - (expert & 7)) % p_x;
-    if (wg_x >= n_x) return;  // padding; uniform over the work-group
-  }
-  const int tile0 = (wg_x * C::kWaves + wave) * C::kWaveTiles;
+  const int tile0 = ((int)blockIdx.x * C::kWaves + wave) * C::kWaveTiles;
   const int n_tg = (count + 7) >> 3;
   const int nq4 = (B + 3) >> 2;
 
@@ -1809,7 +1827,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void gemm_kernel(GemmArg
   for (int t = 0; t < C::kWaveTiles; ++t) {
     const int tile = tile0 + t;
     const bool ok = tile < (int)a.w.tiles;
-    fast = fast && (!ok || fast_raw[t] != 0);
+    fast = fast && (!ok || (fast_raw[t] & kTileFast) != 0);
     const int row = tile * kTileRows + nl;
     // A -0.0 bias becomes +0.0, as the reference's first add does.
     const float b0 = (a.bias != nullptr && ok && row < rows ? bias_raw[t] : 0.0f) + 0.0f;
@@ -1854,7 +1872,499 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void gemm_kernel(GemmArg
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   gemm_epilogue<C, MODE, RESIDUAL, true>(a, tot, n_tg, count, start, tile0, reinterpret_cast<float*>(s_codes0),
-                                   MODE == kDown ? s_slot : nullptr, wg_x);
+                                   MODE == kDown ? s_slot : nullptr);
+}
+
+// ---------------------------------------------------------------------------
+// Expert GEMM of batches whose experts hold many rows: work items of up to 32
+// activation rows on the scaled MFMA v_mfma_scale_f32_32x32x64_f8f6f4.
+//
+// One MFMA covers 32 weight rows x 32 activation rows of one block and part.
+// Its first operand is the block's 32 FP4 codes as stored, with the row's E8M0
+// byte as the hardware's block scale, so no weight is converted; the second
+// holds the activations' codes as two signed digits (q = 16 high + low) in
+// E2M3, digit d as d / 8 (exact up to 15): lanes 0-31 the low digits with
+// block scale 2^3, lanes 32-63 the high digits with 2^7. The weights are the
+// same in both halves of K = 64, so the result is (p / 2) * e8m0, the block's
+// integer dot times its scale: every product is a multiple of 2^-4 below 2^6
+// and the dot has at most 16 significant bits, so nothing rounds in any order
+// (checked against exact sums for every E8M0 byte up to 254, denormal results
+// among them; kTileWide keeps scales whose partial sums could overflow off
+// this path). The MFMA takes 32 cycles for 1,024 dots where the f16 form takes
+// 16 for 256, and its FP4 conversions 16 more.
+//
+// Bound: the float chain, four VALU instructions per 64 (weight row, activation
+// row, block) triples; an f32 instruction takes a SIMD four cycles (the MFMAs
+// run beside them), and the counters show the VALU busy for the whole kernel.
+// So everything else is kept out of the VALU: no weight conversion, weights
+// by DMA and transposed by six swaps a step, one scale register per part. At
+// 2,048 rows of the 20B shape gate_up takes 738 us for 348 M VALU instructions
+// (289 M of them the chain; the two-tile f16 kernel before it 881 us for 424 M
+// with its MFMAs), down 362 us (436); 4,096 rows over 128 experts 1,510 and
+// 744 us (1,835 and 923); 777 rows in Q8 mode 236 and 126 us (324 and 162).
+// Weights straight into registers, read twice by the two halves of a wave, kept
+// the vector-memory path busy for 72% of the Q8 kernel: 283 us.
+//
+// Lane (h, n) holds activation row n and the 16 weight rows 8 k + 4 h + i (k,
+// i < 4) of the wave's 32, and runs their float chains in order; a block's two
+// scales are two registers of the lane. A work-group is eight waves of 32 weight
+// rows sharing the activations; two fit a CU (four waves per SIMD; six-wave
+// work-groups, whose waves fall unevenly on the SIMDs, ran one per CU).
+//
+// Pipeline: steps of four blocks; a step's weights, codes and scales move by
+// DMA into one of two LDS slots while the other is computed, published by one
+// barrier per step; within a step each part's MFMA is issued one part's chain
+// (32 VALU instructions) before its result is read.
+//
+// The gate_up grid's rows (23 work-groups for 5,760 weight rows) are padded to a
+// multiple of 8 and rotated by the item's expert, so tile column x of expert e
+// always runs on XCD (x + e) mod 8 (work-groups reach the XCDs round-robin in
+// launch order): the later chunks of an expert read its weights from the L2
+// that the first one filled. The down grid (12 columns) would leave half of
+// the XCDs a column less of every item and is not padded.
+struct WideCfg {
+  static constexpr int kWaves = 8;
+  static constexpr int kThreads = 64 * kWaves;
+  static constexpr int kWgTiles = 2 * kWaves;
+  static constexpr int kRows = kTileRows * kWgTiles;   // 256
+  static constexpr int kChunk = kHugeChunk;            // 32 activation rows
+  static constexpr int kStep = 4;                      // blocks per step (one group of the v3 layout)
+  static constexpr int kSclSlot = kStep * kChunk * 2;  // floats of a step's activation scales
+  static constexpr int kWSlot = kWaves * 2048;         // a step's weight groups: two 1 KiB groups per wave
+  static_assert(kRows % 64 == 0, "whole 32-value down-input blocks per work-group");
+  static_assert((kStep - 1) * kDigitRecord <= (int)kActSlack, "a last partial step reads inside the slack");
+};
+// Code bytes of a step (operands of one part or two).
+__host__ __device__ constexpr int wide_slot(bool residual) { return (residual ? 2 : 1) * 6144; }
+
+// E8M0 bytes up to which the scaled MFMA's partial sums (below 2^16 * 2^(e -
+// 127)) stay finite.
+constexpr uint32_t kWideScaleHi = 230;
+
+typedef int i32x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+struct WideLoop {
+  __amdgpu_buffer_rsrc_t nib0, nib1, scl, codes, scales;  // the wave's two tiles, its scales, the activations
+  int B, nsteps, nfull4, wave, lane;
+  int vw, vw_tail, vs;      // weight lane offsets: full group, compact last group; scales
+  int vmain, vtail, vscl;   // DMA sources of this lane's code pieces and scale dword in step 0
+};
+
+// The DMA of step q (past the end: the last step again, never used) into one
+// ring slot. Weights: the wave's two 1 KiB groups as stored. Codes: operand o =
+// block * parts + part is one 16-byte lane plane (digit, row) and one tail
+// plane (8 bytes per [row][digit], two operands per instruction); scales
+// [blocks 2 i, 2 i + 1][row][block][part]. Two or three requests per wave and
+// step besides the weights, whichever the wave.
+template <bool RESIDUAL>
+__device__ __forceinline__ uint32_t wide_dma(const WideLoop& k, int q_raw, char* wts, char* codes, float* scl) {
+  constexpr int kParts = RESIDUAL ? 2 : 1, kOps = WideCfg::kStep * kParts, kHalf = kDigitRecord / 2;
+  const int q = min(q_raw, k.nsteps - 1), w = k.wave;
+  const int vw = q < k.nfull4 ? k.vw : k.vw_tail;
+  dma16(k.nib0, wts + w * 2048, vw, q * 1024);
+  dma16(k.nib1, wts + w * 2048 + 1024, vw, q * 1024);
+  const uint32_t ws = __builtin_amdgcn_raw_buffer_load_b32(k.scl, k.vs, q * 64, 0);
+  const int base = q * (WideCfg::kStep * kDigitRecord);
+  if (w < kOps) dma16(k.codes, codes + w * 1024, k.vmain, base + (w / kParts) * kDigitRecord + (w % kParts) * kHalf);
+  const int t = RESIDUAL ? w : w - 4;  // the tail pair this wave moves
+  if (t >= 0 && t < kOps / 2)
+    dma16(k.codes, codes + kOps * 1024 + t * 1024, k.vtail, base + (RESIDUAL ? t : 2 * t) * kDigitRecord);
+  if (w >= 4)
+    dma4(k.scales, reinterpret_cast<char*>(scl) + (w - 4) * 256, k.vscl, q * (WideCfg::kStep * 8) + ((w - 4) >> 1) * 16);
+  return ws;
+}
+
+// The digit (0 low, 1 high) that a lane holds: lanes 0-31 and 32-63 hold one
+// each of every row, swapped for rows 16-31 so that the 8-byte tail reads of 32
+// lanes fall on all LDS banks.
+__device__ __forceinline__ int wide_digit(int lane) { return ((lane >> 5) ^ (lane >> 4)) & 1; }
+
+// Operand o of a step's codes (see wide_dma).
+template <bool RESIDUAL>
+__device__ __forceinline__ i32x8 wide_codes(const char* codes, int j, int part, int lane) {
+  constexpr int kParts = RESIDUAL ? 2 : 1;
+  const int o = j * kParts + part;
+  const u32x4 a = *reinterpret_cast<const u32x4*>(codes + o * 1024 + lane * 16);
+  const u32x2 b = *reinterpret_cast<const u32x2*>(codes + WideCfg::kStep * kParts * 1024 + o * 512 +
+                                                  (lane & 31) * 16 + wide_digit(lane) * 8);
+  return i32x8{(int)a[0], (int)a[1], (int)a[2], (int)a[3], (int)b[0], (int)b[1], 0, 0};
+}
+
+// The four blocks of the lane's weight row (`wl`: the wave's groups at the
+// lane's row; slice s of the row is 256 bytes after slice s - 1, one dword per
+// block): read as stored, in four conflict-free 16-byte reads, and transposed
+// in place by six register swaps, so that w[j] is block j's 32 codes in four
+// consecutive registers. (Reading the dwords of one block 256 bytes apart uses
+// 8 of the 32 LDS banks.)
+__device__ __forceinline__ void wide_swap(uint32_t& a, uint32_t& b) { asm("v_swap_b32 %0, %1" : "+v"(a), "+v"(b)); }
+struct WideW {
+  u32x4 w0, w1, w2, w3;
+};
+__device__ __forceinline__ WideW wide_weights(const char* wl) {
+  const u32x4 a = *reinterpret_cast<const u32x4*>(wl), b = *reinterpret_cast<const u32x4*>(wl + 256);
+  const u32x4 c = *reinterpret_cast<const u32x4*>(wl + 512), d = *reinterpret_cast<const u32x4*>(wl + 768);
+  uint32_t a1 = a[1], a2 = a[2], a3 = a[3], b0 = b[0], b2 = b[2], b3 = b[3], c0 = c[0], c1 = c[1], c3 = c[3],
+           d0 = d[0], d1 = d[1], d2 = d[2];
+  wide_swap(a1, b0);
+  wide_swap(a2, c0);
+  wide_swap(a3, d0);
+  wide_swap(b2, c1);
+  wide_swap(b3, d1);
+  wide_swap(c3, d2);
+  return WideW{u32x4{a[0], a1, a2, a3}, u32x4{b0, b[1], b2, b3}, u32x4{c0, c1, c[2], c3}, u32x4{d0, d1, d2, d[3]}};
+}
+template <int J>
+__device__ __forceinline__ u32x4 wide_pick(u32x4 w0, u32x4 w1, u32x4 w2, u32x4 w3) {
+  if constexpr (J == 0) return w0;
+  else if constexpr (J == 1) return w1;
+  else if constexpr (J == 2) return w2;
+  else return w3;
+}
+
+// cbsz 4: FP4 weights; blgp 2: E2M3 digits; the weights' scale is byte J of the
+// lane's dword (or 1.0), the digits' 2^3 or 2^7 by half.
+template <int J, bool FAST>
+__device__ __forceinline__ f32x16 wide_mfma(u32x4 w, uint32_t ws, i32x8 act, int digit_scale) {
+  const f32x16 zero = {};
+  const i32x8 wv = {(int)w[0], (int)w[1], (int)w[2], (int)w[3], 0, 0, 0, 0};
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wv, act, zero, 4, 2, FAST ? J : 0, FAST ? (int)ws : 127, 0,
+                                                         digit_scale);
+}
+
+// total += d * scale for the lane's 16 weight rows.
+__device__ __forceinline__ void wide_chain(f32x16& tot, const f32x16& d, float scale) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) tot[r] = tot[r] + d[r] * scale;
+}
+
+// A full step on the fast path.
+template <bool RESIDUAL>
+__device__ __forceinline__ void wide_step(f32x16& tot, const char* wl, const char* codes, const float* scl, uint32_t ws,
+                                          int lane) {
+  const int digit_scale = wide_digit(lane) ? 127 + 7 : 127 + 3;
+  const float4* sp = reinterpret_cast<const float4*>(scl) + (lane & 31);
+  const WideW w = wide_weights(wl);
+  i32x8 ap = wide_codes<RESIDUAL>(codes, 0, 0, lane);
+#define GOSSMX_W(J) wide_pick<(J) & 3>(w.w0, w.w1, w.w2, w.w3)
+  if constexpr (RESIDUAL) {
+    i32x8 ar = wide_codes<true>(codes, 0, 1, lane);
+    const float4 s01 = sp[0], s23 = sp[32];  // (block 0 p, r, block 1 p, r), (blocks 2, 3)
+    const float sc[4][2] = {{s01.x, s01.y}, {s01.z, s01.w}, {s23.x, s23.y}, {s23.z, s23.w}};
+    f32x16 dp = wide_mfma<0, true>(GOSSMX_W(0), ws, ap, digit_scale), dr;
+#define GOSSMX_WIDE_BLOCK(J)                                                  \
+  __builtin_amdgcn_sched_barrier(0);                                          \
+  dr = wide_mfma<J, true>(GOSSMX_W(J), ws, ar, digit_scale);                  \
+  if (J < 3) ap = wide_codes<true>(codes, J + 1, 0, lane);                    \
+  __builtin_amdgcn_sched_barrier(0);                                          \
+  wide_chain(tot, dp, sc[J][0]);                                              \
+  __builtin_amdgcn_sched_barrier(0);                                          \
+  if (J < 3) dp = wide_mfma<(J + 1) & 3, true>(GOSSMX_W(J + 1), ws, ap, digit_scale); \
+  if (J < 3) ar = wide_codes<true>(codes, J + 1, 1, lane);                    \
+  __builtin_amdgcn_sched_barrier(0);                                          \
+  wide_chain(tot, dr, sc[J][1]);
+    GOSSMX_WIDE_BLOCK(0)
+    GOSSMX_WIDE_BLOCK(1)
+    GOSSMX_WIDE_BLOCK(2)
+    GOSSMX_WIDE_BLOCK(3)
+#undef GOSSMX_WIDE_BLOCK
+  } else {
+    const float4 s01 = sp[0], s23 = sp[32];
+    const float sc[4] = {s01.x, s01.z, s23.x, s23.z};
+    f32x16 d[2];
+    d[0] = wide_mfma<0, true>(GOSSMX_W(0), ws, ap, digit_scale);
+    ap = wide_codes<false>(codes, 1, 0, lane);
+#define GOSSMX_WIDE_BLOCK(J)                                                             \
+  __builtin_amdgcn_sched_barrier(0);                                                     \
+  if (J < 3) d[(J + 1) & 1] = wide_mfma<(J + 1) & 3, true>(GOSSMX_W(J + 1), ws, ap, digit_scale); \
+  if (J < 2) ap = wide_codes<false>(codes, J + 2, 0, lane);                              \
+  __builtin_amdgcn_sched_barrier(0);                                                     \
+  wide_chain(tot, d[J & 1], sc[J]);
+    GOSSMX_WIDE_BLOCK(0)
+    GOSSMX_WIDE_BLOCK(1)
+    GOSSMX_WIDE_BLOCK(2)
+    GOSSMX_WIDE_BLOCK(3)
+#undef GOSSMX_WIDE_BLOCK
+  }
+#undef GOSSMX_W
+}
+
+// Block J of a step without pipelining: the last partial step, and tiles off
+// the fast path, whose rows' scales come from the lanes that hold them.
+template <bool RESIDUAL, bool FAST, int J>
+__device__ __forceinline__ void wide_block(f32x16& tot, const char* wl, const char* codes, const float* scl,
+                                           uint32_t ws, int lane) {
+  const int digit_scale = wide_digit(lane) ? 127 + 7 : 127 + 3;
+  const float* sp = scl + (J >> 1) * 128 + (lane & 31) * 4 + (J & 1) * 2;
+  float e8[16];
+  if (!FAST) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      e8[r] = e8m0_select((__shfl(ws, 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) >> (8 * J)) & 0xffu);
+  }
+#pragma unroll
+  for (int part = 0; part < (RESIDUAL ? 2 : 1); ++part) {
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(wl) + J;
+    f32x16 d = wide_mfma<J, FAST>(u32x4{p[0], p[64], p[128], p[192]}, ws, wide_codes<RESIDUAL>(codes, J, part, lane), digit_scale);
+    if (!FAST) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) d[r] = d[r] * e8[r];
+    }
+    wide_chain(tot, d, sp[part]);
+  }
+}
+
+template <bool RESIDUAL, bool FAST>
+__device__ __forceinline__ void wide_loop(const WideLoop& k, f32x16& tot, char* w0, char* w1, char* c0, char* c1,
+                                          float* s0, float* s1) {
+  // The lane's row in the wave's weight groups: tile (lane / 16) % 2, row lane % 16.
+  const int wl = k.wave * 2048 + ((k.lane >> 4) & 1) * 1024 + (k.lane & 15) * 16;
+  uint32_t e0, e1;
+  e0 = wide_dma<RESIDUAL>(k, 0, w0, c0, s0);
+#define GOSSMX_STEP(QV, W, C, S, E, NW, NC, NS, NE)                                                      \
+  {                                                                                                      \
+    const int q = (QV);                                                                                  \
+    __builtin_amdgcn_sched_barrier(0);                                                                   \
+    __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8)); /* vmcnt 0: this wave's requests for step q */ \
+    __builtin_amdgcn_s_barrier(); /* ... and every other wave's; the slot of q - 1 is free */            \
+    __builtin_amdgcn_sched_barrier(0);                                                                   \
+    NE = wide_dma<RESIDUAL>(k, q + 1, NW, NC, NS);                                                       \
+    __builtin_amdgcn_sched_barrier(0);                                                                   \
+    const int nb = k.B - 4 * q; /* blocks of the step: 4, fewer in the last one, none past it */         \
+    if (FAST && nb >= 4) {                                                                               \
+      wide_step<RESIDUAL>(tot, W + wl, C, S, E, k.lane);                                                 \
+    } else {                                                                                             \
+      if (nb > 0) wide_block<RESIDUAL, FAST, 0>(tot, W + wl, C, S, E, k.lane);                           \
+      if (nb > 1) wide_block<RESIDUAL, FAST, 1>(tot, W + wl, C, S, E, k.lane);                           \
+      if (nb > 2) wide_block<RESIDUAL, FAST, 2>(tot, W + wl, C, S, E, k.lane);                           \
+      if (nb > 3) wide_block<RESIDUAL, FAST, 3>(tot, W + wl, C, S, E, k.lane);                           \
+    }                                                                                                    \
+    __builtin_amdgcn_sched_barrier(0);                                                                   \
+  }
+  for (int q0 = 0; q0 < k.nsteps; q0 += 2) {
+    GOSSMX_STEP(q0, w0, c0, s0, e0, w1, c1, s1, e1)
+    GOSSMX_STEP(q0 + 1, w1, c1, s1, e1, w0, c0, s0, e0)
+  }
+#undef GOSSMX_STEP
+}
+
+// quantize_q8_block of a block held by four lanes (a quad, eight values each):
+// stores the digit record of the codes, leaves v - q * scale in v and returns
+// the scale. A quad's 32 six-bit codes are six dwords: an even lane's 48 bits
+// and its neighbour's make three, of which it stores the first two.
+__device__ __forceinline__ float wide_quantize(float (&v)[8], int sub, uint8_t* rec, bool store) {
+  float mx = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(v[i]));
+  mx = fmaxf(mx, __uint_as_float(lane_partner<1>(__float_as_uint(mx))));
+  mx = fmaxf(mx, __uint_as_float(lane_partner<2>(__float_as_uint(mx))));
+  const float scale = mx / 127.0f;
+  const float inv = scale == 0.0f ? 0.0f : 1.0f / scale;
+  uint32_t lo0 = 0, lo1 = 0, hi0 = 0, hi1 = 0;  // 48 bits of each digit
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float q = __builtin_amdgcn_fmed3f(round_half_away(v[i] * inv), -127.0f, 127.0f);
+    v[i] = v[i] - q * scale;
+    const uint32_t mag = __float_as_uint(fabsf(q) + 8388608.0f);  // |q| in the low bits (2^23 + |q|)
+    const uint32_t sign = (__float_as_uint(q) >> 31) << 5;
+    const uint32_t lo = (mag & 15u) | sign, hi = ((mag >> 4) & 15u) | sign;
+    if (i < 5) {
+      lo0 |= lo << (6 * i);
+      hi0 |= hi << (6 * i);
+    } else if (i == 5) {
+      lo0 |= lo << 30;
+      hi0 |= hi << 30;
+      lo1 = lo >> 2;
+      hi1 = hi >> 2;
+    } else {
+      lo1 |= lo << (6 * i - 32);
+      hi1 |= hi << (6 * i - 32);
+    }
+  }
+  const bool odd = (sub & 1) != 0;
+  const int first = 3 * (sub >> 1) + (odd ? 2 : 0);  // dword of the digit's six that this lane stores first
+  const uint32_t lo_n = lane_partner<1>(lo0), hi_n = lane_partner<1>(hi0);
+  uint32_t* dst = reinterpret_cast<uint32_t*>(rec);
+  if (store) {
+    // Dword d of a digit: d < 4 at dword d (low) or 4 + d (high), else at 4 + d or 6 + d.
+    const int at = first < 4 ? first : first + 4, high = first < 4 ? 4 : 2;
+    dst[at] = odd ? (lo0 >> 16) | (lo1 << 16) : lo0;
+    dst[at + high] = odd ? (hi0 >> 16) | (hi1 << 16) : hi0;
+    if (!odd) {
+      const int d = first + 1, at2 = d < 4 ? d : d + 4, high2 = d < 4 ? 4 : 2;
+      dst[at2] = lo1 | (lo_n << 16);
+      dst[at2 + high2] = hi1 | (hi_n << 16);
+    }
+  }
+  return scale;
+}
+
+template <int MODE, bool RESIDUAL>
+__global__ __launch_bounds__(WideCfg::kThreads, 4) void gemm_wide_kernel(GemmArgs a) {
+  using C = WideCfg;
+  constexpr int kSlot = wide_slot(RESIDUAL);
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int n = lane & 31, h = lane >> 5;
+  int expert, start, count;
+  if (MODE == kPlain) {
+    expert = a.plain_expert;
+    start = blockIdx.y * C::kChunk;
+    count = min(C::kChunk, a.plain_m - start);
+  } else {
+    const int wi = blockIdx.y;
+    // As gemm_kernel: count and record in one round trip.
+    const int nw = *a.n_work;
+    const int4 rec = reinterpret_cast<const int4*>(a.work)[wi];
+    if ((wi >= nw) | (min(min(rec.x, rec.y), rec.z - 1) < 0)) return;  // uniform over the work-group
+    expert = rec.x;
+    start = rec.y;
+    count = rec.z;
+  }
+  const int rows = (int)a.w.rows, B = (int)a.w.blocks, tiles = (int)a.w.tiles;
+  int wg_x = (int)blockIdx.x;  // tile column
+  if (MODE == kGateUp) {
+    const int n_x = (tiles + C::kWgTiles - 1) / C::kWgTiles;
+    wg_x = (int)blockIdx.x - (expert & 7);
+    if (wg_x < 0) wg_x += (int)gridDim.x;  // n_x padded to a multiple of 8
+    if (wg_x >= n_x) return;  // padding; uniform over the work-group
+  }
+  const int tile0 = wg_x * C::kWgTiles + wave * 2;
+  const int row0 = tile0 * kTileRows;  // the wave's first weight row
+  const int nq4 = (B + 3) >> 2;
+
+  __shared__ int s_row[C::kChunk];
+  __shared__ int s_slot[C::kChunk];
+  constexpr int kValues = C::kRows / 2, kActStride = kValues + 8;  // the epilogue's SwiGLU values (bf16) reuse slot 0
+  constexpr int kSlot0 = kSlot > C::kChunk * kActStride * 2 ? kSlot : C::kChunk * kActStride * 2;
+  __shared__ __align__(16) char s_codes0[kSlot0], s_codes1[kSlot];
+  __shared__ __align__(16) float s_scl0[C::kSclSlot], s_scl1[C::kSclSlot];
+  __shared__ __align__(16) char s_w0[C::kWSlot], s_w1[C::kWSlot];
+  if (tid < C::kChunk) {
+    const int r = start + min(tid, count - 1);  // rows past the item repeat its last one and are never stored
+    s_row[tid] = MODE == kGateUp ? a.route_tok[r] : r;
+    if (MODE != kPlain) s_slot[tid] = a.route_slot[r];
+  }
+
+  WideLoop k;
+  k.B = B;
+  k.nsteps = nq4;
+  k.nfull4 = B >> 2;
+  k.wave = wave;
+  k.lane = lane;
+  // The wave's tiles past the end stream the last one and discard it.
+  const int t0 = min(tile0, tiles - 1), t1 = min(tile0 + 1, tiles - 1);
+  const uint8_t* nib = a.w.nib + (size_t)expert * a.w.nib_stride;
+  k.nib0 = buffer_rsrc(nib + (size_t)t0 * 256 * B);
+  k.nib1 = buffer_rsrc(nib + (size_t)t1 * 256 * B);
+  k.scl = buffer_rsrc(a.w.scl + (size_t)expert * a.w.scl_stride + (size_t)t0 * 64 * nq4);
+  k.vw = lane * 16;
+  k.vw_tail = lane * 4 * (B & 3);
+  k.vs = (n < 16 ? 0 : (t1 - t0) * 64 * nq4) + (n & 15) * 4;
+  const uint8_t* flags = a.w.fast + (size_t)expert * tiles;
+  const int flag = flags[t0] & flags[t1];
+  // Bias rows past the end, or without a bias all of them, are outside the
+  // buffer and read as 0.
+  const __amdgpu_buffer_rsrc_t bias = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(a.bias != nullptr ? a.bias + (size_t)expert * a.bias_expert_stride : nullptr), (short)0,
+      a.bias != nullptr ? rows * 4 : 0, kBufferFlags);
+  f32x16 tot;
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    tot[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(bias, (row0 + 4 * h + 8 * (r >> 2) + (r & 3)) * 4, 0, 0));
+  __syncthreads();
+
+  k.codes = buffer_rsrc(a.actv);
+  k.scales = buffer_rsrc(a.acts);
+  k.vmain = s_row[n] * B * kDigitRecord + wide_digit(lane) * 16;
+  k.vtail = s_row[n] * B * kDigitRecord + 32 + h * (RESIDUAL ? kDigitRecord / 2 : kDigitRecord);
+  k.vscl = (s_row[(lane >> 2) + 16 * (wave & 1)] * B + ((lane >> 1) & 1)) * 8 + (lane & 1) * 4;
+  // A -0.0 bias becomes +0.0, as the reference's first add does.
+#pragma unroll
+  for (int r = 0; r < 16; ++r) tot[r] = tot[r] + 0.0f;
+
+  if (a.fast_ok != 0 && (__builtin_amdgcn_readfirstlane(flag) & kTileWide) != 0)
+    wide_loop<RESIDUAL, true>(k, tot, s_w0, s_w1, s_codes0, s_codes1, s_scl0, s_scl1);
+  else
+    wide_loop<RESIDUAL, false>(k, tot, s_w0, s_w1, s_codes0, s_codes1, s_scl0, s_scl1);
+  // Drain the trailing DMA into the ring before the LDS is reused or the
+  // work-group ends.
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+
+  if (MODE == kPlain || MODE == kDown) {
+    if (n >= count) return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // four consecutive rows
+      const int row = row0 + 8 * q + 4 * h;
+      if (MODE == kDown) {
+        if (row < rows) {  // hidden is a multiple of 32
+          u32x2 v;
+          v[0] = (uint32_t)bf16_bits(tot[4 * q]) | ((uint32_t)bf16_bits(tot[4 * q + 1]) << 16);
+          v[1] = (uint32_t)bf16_bits(tot[4 * q + 2]) | ((uint32_t)bf16_bits(tot[4 * q + 3]) << 16);
+          *reinterpret_cast<u32x2*>(a.y + (size_t)s_slot[n] * rows + row) = v;  // bf16 (cpu_runner.rs:2945-2947)
+        }
+      } else {
+        float* dst = a.out + (size_t)(start + n) * a.out_stride + row;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (row + i < rows) dst[i] = tot[4 * q + i];
+      }
+    }
+  } else {
+    // gate_up epilogue (gemm_epilogue's operations): rows 2 v, 2 v + 1 of the
+    // lane are the (gate, up) pair of value v; the work-group's 64 values per
+    // row meet in LDS as bf16 (they are bf16 values), two 32-value blocks of
+    // the down input.
+    uint16_t* s_act = reinterpret_cast<uint16_t*>(s_codes0);
+    uint16_t sig[8];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) sig[v] = a.sig_tab[swiglu_sigmoid_index(bf16r(tot[2 * v]), a.alpha, a.limit)];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      uint32_t pair = 0;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int v = 2 * q + i;
+        const float gate = bf16r(tot[2 * v]), up = bf16r(tot[2 * v + 1]);
+        const float act = swiglu_finish(gate, up, a.limit, bf16_to_f32(sig[v]));
+        pair |= (__float_as_uint(act) >> 16) << (16 * i);
+        const int row = row0 + 8 * q + 4 * h + 2 * i;
+        if (n < count && row < rows) {
+          if (a.trace_gu != nullptr) {  // CpuExpertTrace::gate_up_projection (bf16 values)
+            a.trace_gu[(size_t)s_slot[n] * rows + row] = gate;
+            a.trace_gu[(size_t)s_slot[n] * rows + row + 1] = up;
+          }
+          if (a.trace_sw != nullptr) a.trace_sw[(size_t)s_slot[n] * (rows / 2) + (row >> 1)] = act;
+        }
+      }
+      *reinterpret_cast<uint32_t*>(s_act + n * kActStride + wave * 16 + 4 * q + 2 * h) = pair;
+    }
+    __syncthreads();
+    // Four lanes per 32-value block, eight values each: quantize_residual_q8
+    // (q8_half_wave's operations) and the digit records.
+    constexpr int kPerRow = C::kRows / 64;
+    const int c = tid / (4 * kPerRow), b = (tid >> 2) % kPerRow, sub = tid & 3, blocks_next = rows / kWgRows;
+    const int blk = wg_x * kPerRow + b;
+    const u32x4 raw = *reinterpret_cast<const u32x4*>(s_act + c * kActStride + b * kBlock + sub * 8);
+    float v[8], zero = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(raw[i] << 16);
+      v[2 * i + 1] = __uint_as_float(raw[i] & 0xffff0000u);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) zero = fmaf(v[i], 0.0f, zero);  // NaN if any value is not finite
+    const bool live = c < count && blk < blocks_next;
+    if (live && zero != zero) atomicOr(a.err, kErrNonFiniteInput);
+    uint8_t* rec = reinterpret_cast<uint8_t*>(a.actv_next) + ((size_t)(start + c) * blocks_next + blk) * kDigitRecord;
+    float2 sc;
+    sc.x = wide_quantize(v, sub, rec, live);
+    sc.y = 0.0f;
+    if (RESIDUAL) sc.y = wide_quantize(v, sub, rec + kDigitRecord / 2, live);
+    if (live && sub == 0) reinterpret_cast<float2*>(a.acts_next)[(size_t)(start + c) * blocks_next + blk] = sc;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2147,7 +2657,7 @@ __global__ __launch_bounds__(64 * 4 * HALVES, HALVES == 2 ? 4 : 2) void gemv_ker
   __builtin_amdgcn_s_waitcnt((kWait & 15) | ((kWait >> 4) << 14) | (7 << 4) | (15 << 8));
   __syncthreads();
 
-  const bool fast = a.fast_ok && fast_raw != 0;
+  const bool fast = a.fast_ok && (fast_raw & kTileFast) != 0;
   // A -0.0 bias becomes +0.0, as the reference's first add does.
   float tot = (a.bias != nullptr && ok && row < rows ? bias_raw : 0.0f) + 0.0f;
   if (HALVES == 1) {
@@ -2295,7 +2805,7 @@ __global__ __launch_bounds__(DownCombineGeom::kThreads, 2) void gemv_down_combin
   __builtin_amdgcn_s_waitcnt(0);  // the image and the ring are in
   __syncthreads();
 
-  const bool fast = live && a.fast_ok && fast_raw != 0;
+  const bool fast = live && a.fast_ok && (fast_raw & kTileFast) != 0;
   // A -0.0 bias becomes +0.0, as the reference's first add does.
   float tot = (live && a.bias != nullptr && row < rows ? bias_raw : 0.0f) + 0.0f;
   if (live) {
@@ -2471,7 +2981,7 @@ __global__ __launch_bounds__(RouteGemvGeom::kThreads, 4) void route_gemv_kernel(
 #pragma unroll
   for (int q = 0; q < R; ++q) gemv_load(L, g0 + q, wn[q], ws[q]);
 
-  const bool fast = a.fast_ok && fast_raw != 0;
+  const bool fast = a.fast_ok && (fast_raw & kTileFast) != 0;
   const float bias = (a.bias != nullptr && ok && row < rows) ? bias_raw : 0.0f;
 
   float* terms = term_base + wave * (Geo::kTermRegion / 4);
@@ -2626,20 +3136,23 @@ __global__ __launch_bounds__(256) void exact_kernel(GemmArgs a) {
   }
 }
 
-// Exactness flag per (expert, tile): 1 when every E8M0 byte of the tile's
-// blocks lies in [kFastScaleLo, kFastScaleHi]. One work-group per tile.
+// Exactness flags per (expert, tile): kTileFast when every E8M0 byte of the
+// tile's blocks lies in [kFastScaleLo, kFastScaleHi], kTileWide when every one
+// is at most kWideScaleHi. One work-group per tile.
 __global__ __launch_bounds__(256) void tile_flags_kernel(TiledWeights w) {
   const size_t e = blockIdx.y, t = blockIdx.x;
   const size_t nq = (w.blocks + 3) / 4;
   const uint8_t* scl = w.scl + e * w.scl_stride + t * 64 * nq;
-  int bad = 0;
+  int bad = 0, over = 0;
   for (size_t i = threadIdx.x; i < kTileRows * w.blocks; i += blockDim.x) {
     const size_t n = i / w.blocks, b = i % w.blocks;
     const uint32_t s = scl[(b / 4) * 64 + n * 4 + (b % 4)];
     bad |= (s - kFastScaleLo) > (kFastScaleHi - kFastScaleLo);
+    over |= s > kWideScaleHi;
   }
   bad = __syncthreads_or(bad);
-  if (threadIdx.x == 0) w.fast[e * w.tiles + t] = bad ? 0 : 1;
+  over = __syncthreads_or(over);
+  if (threadIdx.x == 0) w.fast[e * w.tiles + t] = (uint8_t)((bad ? 0 : kTileFast) | (over ? 0 : kTileWide));
 }
 
 // ---------------------------------------------------------------------------
@@ -2762,9 +3275,15 @@ __global__ __launch_bounds__(256) void prep_records_kernel(const uint8_t* rec, i
     rs = *reinterpret_cast<const float*>(p + 36);
     rq = (int8_t)p[40 + l32];
   }
-  _Float16* dst = act.v + (((size_t)r * blocks + b) * 2) * kBlock;
-  dst[l32] = (_Float16)(float)pq;
-  dst[kBlock + l32] = (_Float16)(float)rq;
+  if (act.digits) {
+    uint8_t* rec = reinterpret_cast<uint8_t*>(act.v) + ((size_t)r * blocks + b) * kDigitRecord;
+    store_digits(rec, (float)pq, l32);
+    if (kind == 2) store_digits(rec + kDigitRecord / 2, (float)rq, l32);
+  } else {
+    _Float16* dst = act.v + (((size_t)r * blocks + b) * 2) * kBlock;
+    dst[l32] = (_Float16)(float)pq;
+    dst[kBlock + l32] = (_Float16)(float)rq;
+  }
   if (l32 == 0) {
     float2 sc;
     sc.x = ps;
@@ -3014,9 +3533,7 @@ hipError_t launch_route_select(const RouteArgs& r, const DispatchArgs& d, int* c
 template <class C>
 static hipError_t launch_gemm_cfg(GemmMode mode, const GemmArgs& a, int grid_work, hipStream_t stream,
                                   hipEvent_t start, hipEvent_t stop) {
-  const unsigned n_x = (unsigned)((a.w.tiles + C::kWgTiles - 1) / C::kWgTiles);
-  const bool pin = C::kPinXcd && mode == kGateUp;
-  const dim3 grid(pin ? (n_x + 7) & ~7u : n_x, (unsigned)grid_work);
+  const dim3 grid((unsigned)((a.w.tiles + C::kWgTiles - 1) / C::kWgTiles), (unsigned)grid_work);
   const dim3 block(C::kThreads);
   auto go = [&](auto kernel) {
     if (start) hipExtLaunchKernelGGL(kernel, grid, block, 0, stream, start, stop, 0, a);
@@ -3038,11 +3555,32 @@ static hipError_t launch_gemm_cfg(GemmMode mode, const GemmArgs& a, int grid_wor
   return hipGetLastError();
 }
 
+static hipError_t launch_gemm_wide(GemmMode mode, const GemmArgs& a, int grid_work, hipStream_t stream,
+                                   hipEvent_t start, hipEvent_t stop) {
+  const unsigned n_x = (unsigned)((a.w.tiles + WideCfg::kWgTiles - 1) / WideCfg::kWgTiles);
+  const dim3 grid(mode == kGateUp ? (n_x + 7) & ~7u : n_x, (unsigned)grid_work);
+  const dim3 block(WideCfg::kThreads);
+  auto go = [&](auto kernel) {
+    if (start) hipExtLaunchKernelGGL(kernel, grid, block, 0, stream, start, stop, 0, a);
+    else hipLaunchKernelGGL(kernel, grid, block, 0, stream, a);
+  };
+  auto pick = [&](auto with, auto without) {
+    if (a.residual) go(with);
+    else go(without);
+  };
+  switch (mode) {
+    case kPlain: pick(gemm_wide_kernel<kPlain, true>, gemm_wide_kernel<kPlain, false>); break;
+    case kGateUp: pick(gemm_wide_kernel<kGateUp, true>, gemm_wide_kernel<kGateUp, false>); break;
+    case kDown: pick(gemm_wide_kernel<kDown, true>, gemm_wide_kernel<kDown, false>); break;
+  }
+  return hipGetLastError();
+}
+
 hipError_t launch_gemm(GemmMode mode, const GemmArgs& a, int chunk, int grid_work, hipStream_t stream,
                        hipEvent_t start, hipEvent_t stop) {
   if (chunk == GemmSmall::kChunk) return launch_gemm_cfg<GemmSmall>(mode, a, grid_work, stream, start, stop);
   if (chunk == GemmBig::kChunk) return launch_gemm_cfg<GemmBig>(mode, a, grid_work, stream, start, stop);
-  if (chunk == GemmHuge::kChunk) return launch_gemm_cfg<GemmHuge>(mode, a, grid_work, stream, start, stop);
+  if (chunk == kHugeChunk) return launch_gemm_wide(mode, a, grid_work, stream, start, stop);
   return hipErrorInvalidValue;
 }
 

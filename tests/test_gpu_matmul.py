@@ -134,6 +134,38 @@ def test_matmul_special_values_and_no_bias(ctx):
     w.close()
 
 
+@pytest.mark.parametrize("kind", [G.ACT_RESIDUAL_Q8, G.ACT_Q8])
+@pytest.mark.parametrize("rows,blocks,m", [(256, 5, 545), (300, 6, 512), (21, 3, 520), (16, 4, 513), (129, 1, 544)])
+def test_wide_items_every_scale_and_extreme_codes(ctx, kind, rows, blocks, m):
+    """The 32-row work items (scaled MFMA): every E8M0 byte, tiles with and
+    without bytes above the scaled range, all codes at their extremes (-128
+    among them), odd tile counts, ragged rows, partial last K groups and last
+    items of 1 and 32 rows."""
+    rng = np.random.default_rng(rows + blocks + m)
+    canonical = O.gen_mxfp4(rows, 3, 1, rows, blocks).reshape(rows, blocks, 17).copy()
+    if rows >= 256:
+        canonical[:256, :, 0] = np.arange(256, dtype=np.uint8)[:, None]
+    else:
+        canonical[:, :, 0] = rng.integers(100, 231, (rows, blocks))
+    canonical[rows // 2:, 0, 1:] = 0x77  # +6 everywhere in the first block
+    canonical = canonical.ravel()
+    act = random_records(rng, m, blocks, kind)
+    part = act["primary"] if kind == G.ACT_RESIDUAL_Q8 else act
+    part["values"][0] = 127
+    part["values"][blocks] = -128
+    part["values"][2 * blocks:3 * blocks] = 0
+    bias = (rng.standard_normal(rows) * 0.1).astype(np.float32)
+    bias[0] = -0.0
+    with np.errstate(all="ignore"):
+        st, want = O.mxfp4_matmul(canonical, rows, blocks, 1, act, m, bias, kind=kind)
+    assert st == O.OK
+    w = G.Weights.upload(ctx, canonical, 1, rows, blocks)
+    got = np.full(m * rows, np.nan, np.float32)
+    G.mxfp4_matmul(ctx, w, 0, act, m, bias, got, kind=kind)
+    assert_same_bits(got, want)
+    w.close()
+
+
 def test_padded_output_columns_are_never_written(ctx):
     # matmul.rs:1121-1165: 1234.0 canaries in the stride padding survive.
     rows, blocks, m, stride = 20, 3, 5, 27

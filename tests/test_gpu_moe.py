@@ -252,7 +252,7 @@ def test_20b_shape_zipf_batch64_all_rows(layer20b):
 
 def test_prefill_2048_all_rows(layer20b):
     """2048 tokens, router computed, several 32-row work items
-    per expert (GemmHuge, two-launch selection): every row."""
+    per expert (the scaled-MFMA geometry, two-launch selection): every row."""
     host, layer = layer20b
     rng = np.random.default_rng(2048)
     x = synth.hidden_rows(rng, 2048)
@@ -319,7 +319,7 @@ def test_120b_shape_zipf_batch256_all_rows(layer120b):
 
 def test_120b_shape_prefill_4096_uniform_all_rows(layer120b):
     """configs[4] prefill: 4096 tokens, near-uniform injected routing over
-    128 experts (16,384 routes, about 128 per expert: GemmHuge and the
+    128 experts (16,384 routes, about 128 per expert: the scaled MFMA and the
     two-launch selection with 64 selection work-groups), every row."""
     host, layer = layer120b
     rng = np.random.default_rng(4096)
