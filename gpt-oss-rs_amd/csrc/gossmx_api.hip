@@ -164,6 +164,7 @@ struct gossmx_layer {
   const gossmx_weights* gate_up = nullptr;
   const gossmx_weights* down = nullptr;
   uint16_t* router_w = nullptr;
+  bool router_exact = false;  // route_exact_matrix of the router weights
   float* router_b = nullptr;
   float* gate_up_bias = nullptr;
   float* down_bias = nullptr;
@@ -980,6 +981,7 @@ int gossmx_layer_create(gossmx_ctx* ctx, const gossmx_moe_config* cfg, const uin
   L->gate_up = gate_up;
   L->down = down;
   L->resident = bytes;
+  L->router_exact = route_exact_matrix(router_weight_bf16, E * H);
   count_transfer(kTransferUpload, bytes);
   hipError_t e = hipMalloc(&L->router_w, E * H * 2);
   if (e == hipSuccess) e = hipMalloc(&L->router_b, E * 4);
@@ -1177,6 +1179,7 @@ static int moe_forward_impl(gossmx_ctx* ctx, const gossmx_layer* L, const gossmx
   ra.x = x;
   ra.router_w = L->router_w;
   ra.router_b = L->router_b;
+  ra.router_exact = L->router_exact ? 1 : 0;
   ra.injected = injected;
   ra.norm_w = route_norm_w;
   ra.norm_eps = norm_eps;

@@ -52,7 +52,7 @@ struct TiledWeights {
   // MFMA's (see tile_flags_kernel); set after every write.
   uint8_t* fast = nullptr;
 };
-constexpr int kTileFast = 1, kTileWide = 2;
+constexpr int kTileWide = 1, kTileFast = 2;  // kTileFast as a threshold: a compare, not a bit test (which waits for the flag early)
 
 // Extra bytes allocated after each plane: the GEMM reads whole 4-block groups
 // (and dword-granular tails) of the last tile unconditionally.
@@ -114,6 +114,7 @@ struct RouteArgs {
   const uint16_t* x;        // [m][hidden] bf16
   const uint16_t* router_w; // [experts][hidden]
   const float* router_b;    // [experts]
+  int router_exact;         // 1: every router weight makes exact products (route_exact_matrix)
   const float* injected;    // [m][experts] or null
   const float* norm_w;      // [hidden] post-attention RMSNorm weight (route_kernel), or null
   float norm_eps;
@@ -159,6 +160,9 @@ constexpr int kRouteGemvExperts = kMaxExperts;
 // Router logits (bf16-rounded, into a.logits) and the gate_up input
 // quantization; followed by one of the two selection paths below.
 hipError_t launch_route(const RouteArgs& a, hipStream_t stream);
+// Whether every bf16 value of w is 0 or far enough from both ends of the
+// exponent range that its products with other such values are exact in f32.
+bool route_exact_matrix(const uint16_t* w, size_t n);
 // Batches past the fused kernel's limits: selection with per-work-group
 // expert counts (cnt: ceil(m / select_rows_per_wg) x experts ints), then the
 // grouping. quantize = 1 adds the gate_up input quantization (no route_kernel).

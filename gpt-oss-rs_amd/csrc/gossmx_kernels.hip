@@ -326,6 +326,8 @@ __device__ __forceinline__ void residual_q8_store_n(const float (&v)[N], const b
 }
 
 // ---------------------------------------------------------------------------
+// The router of rows that route_tile_kernel does not take (hidden sizes past
+// kRouteTileHidden, rows not 16-byte aligned).
 // Router projection and bias with the bf16-rounded logits (the first
 // router_groups work-groups of a row, one per 16 experts; the selection
 // kernels read the logits), and the gate_up input quantization (the rest: 8
@@ -1827,7 +1829,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void gemm_kernel(GemmArg
   for (int t = 0; t < C::kWaveTiles; ++t) {
     const int tile = tile0 + t;
     const bool ok = tile < (int)a.w.tiles;
-    fast = fast && (!ok || (fast_raw[t] & kTileFast) != 0);
+    fast = fast && (!ok || fast_raw[t] >= kTileFast);
     const int row = tile * kTileRows + nl;
     // A -0.0 bias becomes +0.0, as the reference's first add does.
     const float b0 = (a.bias != nullptr && ok && row < rows ? bias_raw[t] : 0.0f) + 0.0f;
@@ -2200,6 +2202,24 @@ __device__ __forceinline__ float wide_quantize(float (&v)[8], int sub, uint8_t* 
   return scale;
 }
 
+// The same with the codes as f16 (gemm_kernel's operand).
+__device__ __forceinline__ float quad_quantize(float (&v)[8], half8& code) {
+  float mx = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(v[i]));
+  mx = fmaxf(mx, __uint_as_float(lane_partner<1>(__float_as_uint(mx))));
+  mx = fmaxf(mx, __uint_as_float(lane_partner<2>(__float_as_uint(mx))));
+  const float scale = mx / 127.0f;
+  const float inv = scale == 0.0f ? 0.0f : 1.0f / scale;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float q = __builtin_amdgcn_fmed3f(round_half_away(v[i] * inv), -127.0f, 127.0f);
+    v[i] = v[i] - q * scale;
+    code[i] = (_Float16)q;
+  }
+  return scale;
+}
+
 template <int MODE, bool RESIDUAL>
 __global__ __launch_bounds__(WideCfg::kThreads, 4) void gemm_wide_kernel(GemmArgs a) {
   using C = WideCfg;
@@ -2364,6 +2384,282 @@ __global__ __launch_bounds__(WideCfg::kThreads, 4) void gemm_wide_kernel(GemmArg
     sc.y = 0.0f;
     if (RESIDUAL) sc.y = wide_quantize(v, sub, rec + kDigitRecord / 2, live);
     if (live && sub == 0) reinterpret_cast<float2*>(a.acts_next)[(size_t)(start + c) * blocks_next + blk] = sc;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Router projection and gate_up input quantization of more than
+// kFusedRouteRows rows (hidden <= kRouteTileHidden): route_kernel's outputs by
+// tiles of rows x experts, so that the rows are read once per expert group
+// instead of the router matrix once per row.
+//
+// A work-group holds its rows in LDS (normalized in place with a.norm_w), quantizes
+// its share of their blocks, and runs the router dots: thread (group, p) owns
+// reduction lanes 2 p and 2 p + 1 (one bf16 pair per 16 elements) of TR rows
+// x TE experts. scalar_bf16_dot's product of two bf16 values is exact in f32
+// when its exponent is far from both ends, so the multiply and the add are one
+// fma with the same bits where every value is 0 or has a magnitude in [2^-60,
+// 2^61) (the router matrix checked when the layer is created, the rows here);
+// otherwise the two instructions.
+//
+// Bound: VALU instructions (28 per 16 dots' steps at TR = 2, TE = 4) and, for
+// small batches, one memory round trip and the 180-step chain. The small tile
+// (4 rows x 8 experts, the whole K range of its experts staged at once) gives
+// small batches work-groups enough; from kRouteSmallGroups of them on the large
+// one (8 x 32, experts by chunks of kRouteTileK) does fewer reads per dot.
+// With the norm: 2,048 rows x 32 experts 48 us (282 us by route_kernel, whose
+// work-groups each re-read 16 experts for one row), 256 x 128 40 us (84);
+// without: 4,096 x 128 149 us (690). Up to 64 rows the two take the same 9-13 us.
+constexpr int kRouteTileHidden = kNormMaxHidden;
+constexpr int kRouteTileK = 256;        // elements of the large tile's expert chunks
+constexpr int kRoutePad = 8;            // dwords after each LDS row: consecutive rows start 8 banks apart
+constexpr int kRouteSmallGroups = 1024;
+constexpr int kRouteQuantShares = 4;    // quantization work-groups per small row tile
+
+// Exponent field in [67, 187], or zero: products of two such values are exact.
+__host__ __device__ constexpr bool route_exact_bf16(uint32_t bits) {
+  return (bits & 0x7fffu) == 0 || ((bits >> 7) & 0xffu) - 67u <= 120u;
+}
+
+// Quantizes one 32-value block held by a quad, eight values per lane
+// (residual_q8_store's operations and stores).
+__device__ __forceinline__ void quad_store(float (&v)[8], int sub, size_t row, int blocks, int blk, const ActBuffers& act,
+                                           int qmode, u32x4 raw) {
+  if (qmode == kProjExactBf16) {
+    reinterpret_cast<u32x4*>(act.v)[(row * blocks + blk) * 4 + sub] = raw;
+    return;
+  }
+  float2 sc;
+  if (act.digits) {
+    uint8_t* rec = reinterpret_cast<uint8_t*>(act.v) + (row * blocks + blk) * kDigitRecord;
+    sc.x = wide_quantize(v, sub, rec, true);
+    sc.y = 0.0f;
+    if (qmode == kProjResidualQ8) sc.y = wide_quantize(v, sub, rec + kDigitRecord / 2, true);
+  } else {
+    half8* dst = reinterpret_cast<half8*>(act.v + (row * blocks + blk) * 2 * kBlock) + sub;
+    half8 q;
+    sc.x = quad_quantize(v, q);
+    dst[0] = q;
+    sc.y = 0.0f;
+    if (qmode == kProjResidualQ8) {
+      sc.y = quad_quantize(v, q);
+    } else {
+      q = half8{};
+    }
+    dst[4] = q;
+  }
+  if (sub == 0) reinterpret_cast<float2*>(act.s)[row * blocks + blk] = sc;
+}
+
+template <int TR, int TE, bool EXACT>
+__device__ __forceinline__ void route_steps(float (&acc)[TR][TE][2], const uint32_t* xs, int xstride, const uint32_t* ws,
+                                            int wstride, int steps) {
+#pragma unroll (TR * TE == 1 ? 18 : 4)
+  for (int k = 0; k < steps; ++k) {
+    uint32_t xd[TR], wd[TE];
+#pragma unroll
+    for (int r = 0; r < TR; ++r) xd[r] = xs[r * xstride + 8 * k];
+#pragma unroll
+    for (int e = 0; e < TE; ++e) wd[e] = ws[e * wstride + 8 * k];
+#pragma unroll
+    for (int e = 0; e < TE; ++e) {
+      const float w0 = __uint_as_float(wd[e] << 16), w1 = __uint_as_float(wd[e] & 0xffff0000u);
+#pragma unroll
+      for (int r = 0; r < TR; ++r) {
+        const float x0 = __uint_as_float(xd[r] << 16), x1 = __uint_as_float(xd[r] & 0xffff0000u);
+        if (EXACT) {
+          acc[r][e][0] = __builtin_fmaf(w0, x0, acc[r][e][0]);
+          acc[r][e][1] = __builtin_fmaf(w1, x1, acc[r][e][1]);
+        } else {
+          acc[r][e][0] = acc[r][e][0] + w0 * x0;
+          acc[r][e][1] = acc[r][e][1] + w1 * x1;
+        }
+      }
+    }
+  }
+}
+
+// Grid (row tiles, expert tiles; small tiles: + kRouteQuantShares), 256 threads: 8 lane pairs x (4 row groups, one
+// per wave) x 8 expert groups; dynamic LDS (route_tile_lds).
+template <int TR, int TE, bool CHUNKED>
+__global__ __launch_bounds__(256) void route_tile_kernel(RouteArgs a) {
+  constexpr int kRows = 4 * TR, kExperts = 8 * TE, kFold = 17;
+  extern __shared__ __align__(16) uint32_t s_tile[];
+  __shared__ float s_part[kRows][16];
+  __shared__ float s_inv[kRows];
+  const int tid = threadIdx.x, p = tid & 7, eg = (tid >> 3) & 7, rg = tid >> 6;
+  const int H = a.hidden, E = a.experts, xstride = H / 2 + kRoutePad;
+  const int wlen = CHUNKED ? kRouteTileK : H, wstride = wlen / 2 + kRoutePad;
+  const int r0 = (int)blockIdx.x * kRows, e0 = (int)blockIdx.y * kExperts;
+  const int n_experts = (E + kExperts - 1) / kExperts;
+  const bool quant_only = !CHUNKED && (int)blockIdx.y >= n_experts;
+  uint32_t* xs = s_tile;
+  uint32_t* ws = s_tile + kRows * xstride;
+  const int pieces = H / 8;  // 16-byte pieces per row
+
+  // Wave w stages rows and experts w, w + 4, ... (past the batch or the last
+  // expert: the last one again), kBatch pieces per lane of each in flight.
+  constexpr int kBatch = 6, kWaveExperts = CHUNKED ? 0 : kExperts / 4;
+  const int wave = tid >> 6, lane = tid & 63;
+  for (int c0 = lane; c0 < pieces; c0 += 64 * kBatch) {
+    u32x4 xv[TR][kBatch], wv[kWaveExperts + 1][kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int c = min(c0 + 64 * i, pieces - 1);
+#pragma unroll
+      for (int r = 0; r < TR; ++r)
+        xv[r][i] = reinterpret_cast<const u32x4*>(a.x + (size_t)min(r0 + wave + 4 * r, a.m - 1) * H)[c];
+#pragma unroll
+      for (int e = 0; e < kWaveExperts; ++e)
+        if (!quant_only) wv[e][i] = reinterpret_cast<const u32x4*>(a.router_w + (size_t)min(e0 + wave + 4 * e, E - 1) * H)[c];
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int c = min(c0 + 64 * i, pieces - 1);
+#pragma unroll
+      for (int r = 0; r < TR; ++r) *reinterpret_cast<u32x4*>(xs + (wave + 4 * r) * xstride + c * 4) = xv[r][i];
+#pragma unroll
+      for (int e = 0; e < kWaveExperts; ++e)
+        if (!quant_only) *reinterpret_cast<u32x4*>(ws + (wave + 4 * e) * wstride + c * 4) = wv[e][i];
+    }
+  }
+  __syncthreads();
+  if (a.norm_w) {
+    // row_inverse_rms's operations: lane l sums x_i * x_i over i = l mod 16, the
+    // lanes are added 0..15.
+    for (int v = tid; v < kRows * 8; v += 256) {
+      const int r = v >> 3, l = v & 7;
+      const uint32_t* row = xs + r * xstride + l;
+      float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll 6
+      for (int k = 0; k < H / 16; ++k) {
+        const uint32_t d = row[8 * k];
+        const float lo = __uint_as_float(d << 16), hi = __uint_as_float(d & 0xffff0000u);
+        s0 = s0 + lo * lo;
+        s1 = s1 + hi * hi;
+      }
+      s_part[r][2 * l] = s0;
+      s_part[r][2 * l + 1] = s1;
+    }
+    __syncthreads();
+    if (tid < kRows) {
+      float ss = -0.0f;
+      for (int l = 0; l < 16; ++l) ss = ss + s_part[tid][l];
+      s_inv[tid] = 1.0f / sqrtf(ss / (float)H + a.norm_eps);
+    }
+    __syncthreads();
+  }
+  // Normalization in place (norm_boundary) and the check of the rows' exponents.
+  int inexact = a.router_exact ? 0 : 1;
+  for (int c0 = lane; c0 < pieces; c0 += 64 * kBatch) {
+    float4 nw[kBatch][2];
+    if (a.norm_w) {
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const float4* n = reinterpret_cast<const float4*>(a.norm_w) + 2 * min(c0 + 64 * i, pieces - 1);
+        nw[i][0] = n[0];
+        nw[i][1] = n[1];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < TR; ++r) {
+      const float inv = a.norm_w ? s_inv[wave + 4 * r] : 1.0f;
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        if (c0 + 64 * i >= pieces) continue;
+        u32x4* at = reinterpret_cast<u32x4*>(xs + (wave + 4 * r) * xstride + (c0 + 64 * i) * 4);
+        u32x4 d = *at;
+        if (a.norm_w) {
+          const float w[8] = {nw[i][0].x, nw[i][0].y, nw[i][0].z, nw[i][0].w,
+                              nw[i][1].x, nw[i][1].y, nw[i][1].z, nw[i][1].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float lo = __uint_as_float(d[q] << 16), hi = __uint_as_float(d[q] & 0xffff0000u);
+            d[q] = (uint32_t)bf16_bits(lo * inv * w[2 * q]) | ((uint32_t)bf16_bits(hi * inv * w[2 * q + 1]) << 16);
+          }
+          *at = d;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) inexact |= !route_exact_bf16(d[q] & 0xffffu) | !route_exact_bf16(d[q] >> 16);
+      }
+    }
+  }
+  const bool exact = __syncthreads_or(inexact) == 0;
+
+  // Share qi of qn of the rows' blocks: large tiles split them over the expert
+  // tiles, small ones leave them to work-groups of their own, which run beside
+  // the router's.
+  const int qn = CHUNKED ? (int)gridDim.y : kRouteQuantShares, qi = CHUNKED ? (int)blockIdx.y : (int)blockIdx.y - n_experts;
+  if (a.quant && qi >= 0) {
+    const int blocks = H / kBlock, sub = tid & 3, nq = (blocks - qi + qn - 1) / qn;
+    for (int v = tid >> 2; v < min(kRows, a.m - r0) * nq; v += 64) {  // uniform per quad
+      const int r = v / nq, b = (v - r * nq) * qn + qi;
+      const u32x4 raw = *reinterpret_cast<const u32x4*>(xs + r * xstride + b * (kBlock / 2) + sub * 4);
+      float val[8], zero = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        val[2 * q] = __uint_as_float(raw[q] << 16);
+        val[2 * q + 1] = __uint_as_float(raw[q] & 0xffff0000u);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) zero = fmaf(val[q], 0.0f, zero);  // NaN if any value is not finite
+      // The exact-BF16 projection takes its input unchecked (prepare_expert_input, cpu_runner.rs:3108).
+      if (a.qmode != kProjExactBf16 && zero != zero) atomicOr(a.err, kErrNonFiniteInput);
+      quad_store(val, sub, (size_t)(r0 + r), blocks, b, a.act, a.qmode, raw);
+    }
+  }
+
+  if (quant_only) return;  // uniform over the work-group
+
+  float acc[TR][TE][2] = {};
+  const uint32_t* xt = xs + rg * xstride + p;  // rows rg, rg + 4, ...
+  const uint32_t* wt = ws + eg * wstride + p;  // experts eg, eg + 8, ...
+  if (CHUNKED) {
+    constexpr int kPieces = kExperts * kRouteTileK / 8 / 256;  // pieces per thread and chunk
+    u32x4 next[kPieces];
+    auto fetch = [&](int c0) {
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) {
+        const int v = tid + 256 * i, e = v / (kRouteTileK / 8), c = v % (kRouteTileK / 8);
+        next[i] = reinterpret_cast<const u32x4*>(a.router_w + (size_t)min(e0 + e, E - 1) * H)[min(c0 / 8 + c, pieces - 1)];
+      }
+    };
+    fetch(0);
+    for (int c0 = 0; c0 < H; c0 += kRouteTileK) {  // uniform
+      __syncthreads();  // the previous chunk's readers are done
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) {
+        const int v = tid + 256 * i, e = v / (kRouteTileK / 8), c = v % (kRouteTileK / 8);
+        *reinterpret_cast<u32x4*>(ws + e * wstride + c * 4) = next[i];
+      }
+      __syncthreads();
+      if (c0 + kRouteTileK < H) fetch(c0 + kRouteTileK);
+      const int steps = min(kRouteTileK, H - c0) / 16;
+      if (exact) route_steps<TR, TE, true>(acc, xt + c0 / 2, 4 * xstride, wt, 8 * wstride, steps);
+      else route_steps<TR, TE, false>(acc, xt + c0 / 2, 4 * xstride, wt, 8 * wstride, steps);
+    }
+  } else {
+    if (exact) route_steps<TR, TE, true>(acc, xt, 4 * xstride, wt, 8 * wstride, H / 16);
+    else route_steps<TR, TE, false>(acc, xt, 4 * xstride, wt, 8 * wstride, H / 16);
+  }
+  __syncthreads();  // the experts' LDS is free: the lane sums [row][expert][lane]
+  float* fold = reinterpret_cast<float*>(ws);
+#pragma unroll
+  for (int r = 0; r < TR; ++r)
+#pragma unroll
+    for (int e = 0; e < TE; ++e) {
+      float* f = fold + ((rg + 4 * r) * kExperts + eg + 8 * e) * kFold + 2 * p;
+      f[0] = acc[r][e][0];
+      f[1] = acc[r][e][1];
+    }
+  __syncthreads();
+  for (int v = tid; v < kRows * kExperts; v += 256) {
+    const int r = r0 + v / kExperts, e = e0 + v % kExperts;
+    if (r < a.m && e < E) {
+      float s = fold[v * kFold];
+      for (int j = 1; j < 16; ++j) s = s + fold[v * kFold + j];
+      a.logits[(size_t)r * E + e] = bf16r(s + a.router_b[e]);  // += bias (cpu_runner.rs:2781-2783), bf16 (:2829)
+    }
   }
 }
 
@@ -2657,7 +2953,7 @@ __global__ __launch_bounds__(64 * 4 * HALVES, HALVES == 2 ? 4 : 2) void gemv_ker
   __builtin_amdgcn_s_waitcnt((kWait & 15) | ((kWait >> 4) << 14) | (7 << 4) | (15 << 8));
   __syncthreads();
 
-  const bool fast = a.fast_ok && (fast_raw & kTileFast) != 0;
+  const bool fast = a.fast_ok && fast_raw >= kTileFast;
   // A -0.0 bias becomes +0.0, as the reference's first add does.
   float tot = (a.bias != nullptr && ok && row < rows ? bias_raw : 0.0f) + 0.0f;
   if (HALVES == 1) {
@@ -2805,7 +3101,7 @@ __global__ __launch_bounds__(DownCombineGeom::kThreads, 2) void gemv_down_combin
   __builtin_amdgcn_s_waitcnt(0);  // the image and the ring are in
   __syncthreads();
 
-  const bool fast = live && a.fast_ok && (fast_raw & kTileFast) != 0;
+  const bool fast = live && a.fast_ok && fast_raw >= kTileFast;
   // A -0.0 bias becomes +0.0, as the reference's first add does.
   float tot = (live && a.bias != nullptr && row < rows ? bias_raw : 0.0f) + 0.0f;
   if (live) {
@@ -2981,7 +3277,7 @@ __global__ __launch_bounds__(RouteGemvGeom::kThreads, 4) void route_gemv_kernel(
 #pragma unroll
   for (int q = 0; q < R; ++q) gemv_load(L, g0 + q, wn[q], ws[q]);
 
-  const bool fast = a.fast_ok && (fast_raw & kTileFast) != 0;
+  const bool fast = a.fast_ok && fast_raw >= kTileFast;
   const float bias = (a.bias != nullptr && ok && row < rows) ? bias_raw : 0.0f;
 
   float* terms = term_base + wave * (Geo::kTermRegion / 4);
@@ -3469,9 +3765,40 @@ __global__ void selftest_kernel(float* out) {
 
 static inline unsigned grid1d(size_t n, unsigned block) { return (unsigned)((n + block - 1) / block); }
 
+static size_t route_tile_lds(int hidden, int rows, int experts, int wlen) {
+  const size_t w = (size_t)experts * (wlen * 2 + kRoutePad * 4), fold = (size_t)rows * experts * 17 * 4;
+  return (size_t)rows * (hidden * 2 + kRoutePad * 4) + std::max(w, fold);
+}
+
+bool route_exact_matrix(const uint16_t* w, size_t n) {
+  // route_exact_bf16 in 16-bit operations, which vectorize.
+  uint16_t bad = 0;
+  for (size_t i = 0; i < n; ++i) {
+    const uint16_t mag = w[i] & 0x7fffu, above = (uint16_t)(mag - (67u << 7));
+    bad |= (uint16_t)((mag != 0) & (above > (uint16_t)((121u << 7) - 1u)));
+  }
+  return bad == 0;
+}
+
 hipError_t launch_route(const RouteArgs& a, hipStream_t stream) {
-  const int quant_groups = a.quant ? (a.hidden / kBlock + kRouteQuantBlocks - 1) / kRouteQuantBlocks : 0;
   if (a.hidden % 32 != 0 || a.experts > kMaxExperts) return hipErrorInvalidValue;
+  const auto a16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (a.hidden <= kRouteTileHidden && a16(a.x) && a16(a.norm_w)) {
+    // Small tiles while their experts' whole K range fits and they are few.
+    const size_t lds_small = route_tile_lds(a.hidden, 4, 8, a.hidden), limit = 152 * 1024;
+    const dim3 small((a.m + 3) / 4, (a.experts + 7) / 8), large((a.m + 7) / 8, (a.experts + 31) / 32);
+    if (lds_small <= limit && small.x * small.y <= (unsigned)kRouteSmallGroups) {
+      const dim3 grid(small.x, small.y + (a.quant ? kRouteQuantShares : 0));
+      hipLaunchKernelGGL((route_tile_kernel<1, 1, false>), grid, dim3(256), (unsigned)lds_small, stream, a);
+      return hipGetLastError();
+    }
+    const size_t lds_large = route_tile_lds(a.hidden, 8, 32, kRouteTileK);
+    if (lds_large <= limit) {
+      hipLaunchKernelGGL((route_tile_kernel<2, 4, true>), large, dim3(256), (unsigned)lds_large, stream, a);
+      return hipGetLastError();
+    }
+  }
+  const int quant_groups = a.quant ? (a.hidden / kBlock + kRouteQuantBlocks - 1) / kRouteQuantBlocks : 0;
   hipLaunchKernelGGL(route_kernel, dim3(a.m, router_groups(a) + quant_groups), dim3(256), 0, stream, a);
   return hipGetLastError();
 }

@@ -289,6 +289,38 @@ def test_routing_paths_bit_exact(ctx, experts, top_k, m, inject):
     close(layer)
 
 
+@pytest.mark.parametrize("experts,hidden,m,norm,shrink", [
+    (3, 32, 5, False, 0), (31, 96, 6, True, 0), (33, 4096, 9, True, 0), (128, 2880, 37, False, 0),
+    (8, 64, 4101, True, 0),      # large tiles, ragged last row tile
+    (40, 320, 2051, False, 0),   # large tiles, two expert tiles, a partial K chunk
+    (8, 96, 21, False, 64),      # products below f32's exact range: multiply and add apart
+    (8, 64, 4101, False, 64),
+])
+def test_router_tiles_bit_exact(ctx, experts, hidden, m, norm, shrink):
+    """The tiled router (4 x 8 and 8 x 32 tiles): logits, routing and the
+    quantized input's products against the oracle at the tiles' edges, and
+    with rows and router weights of about 2^-64, whose products round."""
+    host = O.synthetic_layer(41, 0, experts=experts, hidden=hidden, intermediate=32, top_k=2)
+    x = O.gen_hidden(41, 500 + m, m, hidden)
+    if shrink:
+        host.router_weight = synth.bf16_bits(synth.bf16_to_f32(host.router_weight) * np.float32(2.0 ** -shrink))
+        host.router_bias = np.zeros_like(host.router_bias)
+        x = synth.bf16_bits(synth.bf16_to_f32(x) * np.float32(2.0 ** -shrink))
+    layer = gpu_layer(ctx, host)
+    if norm:
+        w = (1.0 + 0.25 * np.random.default_rng(m).standard_normal(hidden)).astype(np.float32)
+        want = O.moe_batch(host, O.norm_boundary(x, w, 1e-5))
+        got = layer.forward_residual(x, w, 1e-5)
+    else:
+        want = O.moe_batch(host, x)
+        got = layer.forward(x)
+    assert want["status"] == O.OK
+    assert_moe_equal(got, want)
+    if shrink:
+        assert (want["router_logits"] != 0).any()
+    close(layer)
+
+
 @pytest.fixture(scope="module")
 def layer120b(ctx):
     host = O.synthetic_layer(120, 0, experts=128)
