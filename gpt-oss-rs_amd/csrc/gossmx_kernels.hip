@@ -3347,88 +3347,216 @@ __global__ __launch_bounds__(RouteGemvGeom::kThreads, 4) void route_gemv_kernel(
 // the input values k = l mod 16 in increasing k, multiply then add
 // (accumulate_mxfp4_bf16_block, lib.rs:932-945: value v of a block feeds lane
 // v % 16, so lane l takes k = 32 b + l, then 32 b + l + 16, block after
-// block). A conformance path, VALU only: a work-group is one 16-row weight
-// tile x 16 lanes (one thread per row and lane) over one work item of the
-// dispatch's list (at most kChunkMax routes, one accumulator each).
-// gate_up: bf16 round trip, SwiGLU pairs (rows 2i, 2i + 1 of the tile) into
-// the down input [grouped route][rows / 2] bf16; down: y [slot][rows] bf16.
+// block). VALU only. A work-group is 64 weight rows x one work item of the
+// dispatch's list, in passes of up to 8 routes: their input rows go to LDS as
+// bf16, thread (group, p) owns lanes 2 p and 2 p + 1 of two weight rows (one
+// byte of two of a block's dwords each) and every route of the pass, and keeps
+// the next four blocks' weights in flight.
+// gate_up: bf16 round trip, SwiGLU pairs (rows 2i, 2i + 1) into the down input
+// [grouped route][rows / 2] bf16; down: y [slot][rows] bf16.
+//
+// A weight is a bf16 value with two significant bits and x a bf16 value, so
+// where their exponents are far from both ends (the tiles' scales in
+// kTileFast's range, the inputs by route_exact_bf16) the product is exact and
+// multiply and add are one fma with the same bits, on weights converted with
+// their scale by v_cvt_scalef32_pk_f32_fp4. Elsewhere: unscaled weights, e8m0,
+// bf16 and both instructions.
+//
+// Bound: VALU, 4 T fmas, T unpacks of x and 2 conversions per row and block for
+// T routes (128 rows per work-group at two waves per SIMD ran 4% slower). The
+// whole block at 40 rows of the 20B shape takes 323 us, 2,166 us with the
+// kernel before it, which read every input value from global memory for each
+// weight row; 1 row 56 / 211 us, 300 rows 1,522 / 11,340 us.
 
-__constant__ float kE2M1[16] = {0.0f,  0.5f,  1.0f,  1.5f,  2.0f,  3.0f,  4.0f,  6.0f,
-                                -0.0f, -0.5f, -1.0f, -1.5f, -2.0f, -3.0f, -4.0f, -6.0f};
+constexpr int kExactRows = 64;    // weight rows per work-group
+constexpr int kExactRoutes = 8;   // routes per pass
+constexpr int kExactTN = kExactRows / 32;
+constexpr int kExactFold = 4;     // routes folded at once
+constexpr int kExactPad = 8;      // dwords after each input row in LDS
+
+// Four blocks of one weight row: slices p / 4 and 2 + p / 4, and the scales.
+struct ExactW {
+  u32x4 lo, hi;
+  uint32_t s;
+};
+
+template <int T, bool EXACT>
+__device__ __forceinline__ void exact_group(float (&acc)[kExactTN][T][2], const ExactW (&w)[kExactTN], const uint32_t* xs,
+                                            int xstride, int nb, int byte) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (j >= nb) break;
+    float wv[kExactTN][4];
+#pragma unroll
+    for (int n = 0; n < kExactTN; ++n) {
+      const uint32_t c = (((w[n].lo[j] >> byte) & 0xffu) | (((w[n].hi[j] >> byte) & 0xffu) << 8));
+      const uint32_t sb = (w[n].s >> (8 * j)) & 0xffu;
+      const float scale = EXACT ? __uint_as_float(sb << 23) : 1.0f;
+      const auto a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 0);
+      const auto b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 1);
+      wv[n][0] = a[0];
+      wv[n][1] = a[1];
+      wv[n][2] = b[0];
+      wv[n][3] = b[1];
+      if (!EXACT) {
+        const float e8 = e8m0_select(sb);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wv[n][i] = bf16r(wv[n][i] * e8);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      if (t % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+      const uint32_t d0 = xs[t * xstride + j * 16], d1 = xs[t * xstride + j * 16 + 8];
+      const float x0 = __uint_as_float(d0 << 16), x1 = __uint_as_float(d0 & 0xffff0000u);
+      const float x2 = __uint_as_float(d1 << 16), x3 = __uint_as_float(d1 & 0xffff0000u);
+#pragma unroll
+      for (int n = 0; n < kExactTN; ++n) {
+        float (&c)[2] = acc[n][t];
+        if (EXACT) {
+          c[0] = __builtin_fmaf(wv[n][0], x0, c[0]);
+          c[1] = __builtin_fmaf(wv[n][1], x1, c[1]);
+          c[0] = __builtin_fmaf(wv[n][2], x2, c[0]);
+          c[1] = __builtin_fmaf(wv[n][3], x3, c[1]);
+        } else {
+          c[0] = c[0] + wv[n][0] * x0;
+          c[1] = c[1] + wv[n][1] * x1;
+          c[0] = c[0] + wv[n][2] * x2;
+          c[1] = c[1] + wv[n][3] * x3;
+        }
+      }
+    }
+  }
+}
+
+template <int MODE, int T>
+__device__ __forceinline__ void exact_pass(const GemmArgs& a, int expert, int start, int count, uint32_t* xs, float* fold) {
+  const int tid = threadIdx.x, p = tid & 7, group = tid >> 3;
+  const int rows = (int)a.w.rows, B = (int)a.w.blocks, K = B * kBlock, tiles = (int)a.w.tiles;
+  const int nq4 = (B + 3) >> 2, xstride = K / 2 + kExactPad;
+  const int row0 = (int)blockIdx.x * kExactRows;
+  // The pass's input rows (past the item: its last one again).
+  int inexact = a.fast_ok ? 0 : 1;
+  for (int t = tid >> 5; t < T; t += 8) {
+    const int r = start + min(t, count - 1);
+    const uint16_t* src = a.xin + (size_t)(MODE == kGateUp ? a.route_tok[r] : r) * K;
+    const bool aligned = (reinterpret_cast<uintptr_t>(a.xin) & 15) == 0;  // the caller's rows may not be
+#pragma unroll 4
+    for (int c = tid & 31; c < K / 8; c += 32) {
+      u32x4 d;
+      if (aligned) {
+        d = reinterpret_cast<const u32x4*>(src)[c];
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[q] = (uint32_t)src[c * 8 + 2 * q] | ((uint32_t)src[c * 8 + 2 * q + 1] << 16);
+      }
+      *reinterpret_cast<u32x4*>(xs + t * xstride + c * 4) = d;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) inexact |= !route_exact_bf16(d[q] & 0xffffu) | !route_exact_bf16(d[q] >> 16);
+    }
+  }
+  if (tid < kExactRows / kTileRows)
+    inexact |= a.w.fast[(size_t)expert * tiles + min(row0 / kTileRows + tid, tiles - 1)] < kTileFast;
+  const bool exact = __syncthreads_or(inexact) == 0;
+
+  // Weight rows group + 32 n (past the end: the last tile's).
+  const __amdgpu_buffer_rsrc_t nib = buffer_rsrc(a.w.nib + (size_t)expert * a.w.nib_stride);
+  const __amdgpu_buffer_rsrc_t scl = buffer_rsrc(a.w.scl + (size_t)expert * a.w.scl_stride);
+  const int g = p >> 2, byte = 8 * (p & 3), nr = group % kTileRows;  // the rows have one place in their tiles
+  int tile[kExactTN];
+#pragma unroll
+  for (int n = 0; n < kExactTN; ++n) tile[n] = min((row0 + group + 32 * n) / kTileRows, tiles - 1);
+  auto fetch = [&](int q, ExactW (&w)[kExactTN]) {
+    // The compact last group holds nb dwords per lane; the 16 bytes read there
+    // end inside the tile or the plane slack, and dwords past nb are not used.
+    const int nb = min(4, B - 4 * q);
+#pragma unroll
+    for (int n = 0; n < kExactTN; ++n) {
+      const int at = tile[n] * 256 * B + (g * 16 + nr) * nb * 4;
+      w[n].lo = __builtin_amdgcn_raw_buffer_load_b128(nib, at, q * 1024, 0);
+      w[n].hi = __builtin_amdgcn_raw_buffer_load_b128(nib, at, q * 1024 + 128 * nb, 0);
+      w[n].s = __builtin_amdgcn_raw_buffer_load_b32(scl, tile[n] * 64 * nq4 + nr * 4, q * 64, 0);
+    }
+  };
+  float acc[kExactTN][T][2] = {};
+  ExactW cur[kExactTN], next[kExactTN];
+  fetch(0, cur);
+#pragma unroll 1
+  for (int q = 0; q < nq4; ++q) {
+    fetch(min(q + 1, nq4 - 1), next);
+    const int nb = min(4, B - 4 * q);
+    if (exact) exact_group<T, true>(acc, cur, xs + p + q * 64, xstride, nb, byte);
+    else exact_group<T, false>(acc, cur, xs + p + q * 64, xstride, nb, byte);
+#pragma unroll
+    for (int n = 0; n < kExactTN; ++n) cur[n] = next[n];
+  }
+
+  // kExactFold routes at a time: the lane sums [route][row][lane] in LDS, folded
+  // in lane order from -0.0, then the bias.
+  constexpr int kF = T < kExactFold ? T : kExactFold, kLane = 17;
+  __syncthreads();  // every thread is done with the input rows
+  float* s_gu = fold + kF * kExactRows * kLane;  // [route][row] bf16 values (gate_up)
+#pragma unroll 1
+  for (int t0 = 0; t0 < T && t0 < count; t0 += kF) {  // uniform
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      if (u < t0 || u >= t0 + kF) continue;
+#pragma unroll
+      for (int n = 0; n < kExactTN; ++n) {
+        float* f = fold + ((u - t0) * kExactRows + group + 32 * n) * kLane + 2 * p;
+        f[0] = acc[n][u][0];
+        f[1] = acc[n][u][1];
+      }
+    }
+    __syncthreads();
+    for (int v = tid; v < kF * kExactRows; v += 256) {
+      const int u = v / kExactRows, row = row0 + v % kExactRows, t = t0 + u;
+      if (t >= count || row >= rows) continue;
+      float sum = -0.0f;
+#pragma unroll
+      for (int l = 0; l < 16; ++l) sum = sum + fold[v * kLane + l];
+      const float total = (a.bias != nullptr ? a.bias[(size_t)expert * a.bias_expert_stride + row] : 0.0f) + sum;
+      if (MODE == kDown) {
+        a.y[(size_t)a.route_slot[start + t] * rows + row] = bf16_bits(total);  // bf16 (cpu_runner.rs:2945-2947)
+      } else {
+        const float gu = bf16r(total);  // bf16 (cpu_runner.rs:2905)
+        s_gu[v] = gu;
+        if (a.trace_gu != nullptr) a.trace_gu[(size_t)a.route_slot[start + t] * rows + row] = gu;
+      }
+    }
+    __syncthreads();
+    if (MODE == kGateUp) {
+      for (int v = tid; v < kF * kExactRows / 2; v += 256) {
+        const int u = v / (kExactRows / 2), i = v % (kExactRows / 2), t = t0 + u, half = rows / 2;
+        if (t >= count || row0 / 2 + i >= half) continue;
+        const float act = swiglu_one(s_gu[u * kExactRows + 2 * i], s_gu[u * kExactRows + 2 * i + 1], a.alpha, a.limit, a.sig_tab);
+        a.act_next16[(size_t)(start + t) * half + row0 / 2 + i] = bf16_bits(act);  // activated_bf16 (cpu_runner.rs:2917)
+        if (a.trace_sw != nullptr) a.trace_sw[(size_t)a.route_slot[start + t] * half + row0 / 2 + i] = act;
+      }
+    }
+  }
+  __syncthreads();  // the LDS is free for the next pass
+}
+
+// Dynamic LDS: the input rows; the fold buffers reuse it after the K loop.
+static size_t exact_lds(size_t K, int routes) {
+  const size_t in = (size_t)routes * (K / 2 + kExactPad) * 4;
+  return std::max(in, (size_t)std::min(routes, kExactFold) * kExactRows * 18 * 4);
+}
 
 template <int MODE>
-__global__ __launch_bounds__(256) void exact_kernel(GemmArgs a) {
-  const int tid = threadIdx.x, nn = tid >> 4, l = tid & 15;
+__global__ __launch_bounds__(256, 3) void exact_kernel(GemmArgs a, int routes) {
+  extern __shared__ __align__(16) uint32_t s_exact[];
   const int wi = blockIdx.y;
   const int nw = *a.n_work;
   const int4 rec = reinterpret_cast<const int4*>(a.work)[wi];
   if (wi >= nw) return;  // uniform over the work-group
-  const int expert = rec.x, start = rec.y, count = rec.z;
-  const int rows = (int)a.w.rows, B = (int)a.w.blocks, K = B * kBlock;
-  const int tile = blockIdx.x, n = tile * kTileRows + nn;
-  const int nq4 = (B + 3) >> 2;
-  const uint8_t* nib = a.w.nib + (size_t)expert * a.w.nib_stride + (size_t)tile * 256 * B;
-  const uint8_t* scl = a.w.scl + (size_t)expert * a.w.scl_stride + (size_t)tile * 64 * nq4;
-  __shared__ const uint16_t* s_in[kChunkMax];
-  if (tid < kChunkMax) {
-    const int t = min(tid, count - 1);
-    const size_t src = MODE == kGateUp ? (size_t)a.route_tok[start + t] : (size_t)(start + t);
-    s_in[tid] = a.xin + src * K;
-  }
-  __syncthreads();
-  float acc[kChunkMax];
-#pragma unroll
-  for (int t = 0; t < kChunkMax; ++t) acc[t] = 0.0f;
-  const int g_lo = l >> 3, shift = 4 * (l & 7);
-  for (int b = 0; b < B; ++b) {
-    const int q = b >> 2, j = b & 3, nb = min(4, B - 4 * q);
-    // Codes l and l + 16 of row nn: k-slices l / 8 and 2 + l / 8 of the group.
-    const uint32_t d0 = *reinterpret_cast<const uint32_t*>(nib + q * 1024 + (g_lo * 16 + nn) * nb * 4 + j * 4);
-    const uint32_t d1 = *reinterpret_cast<const uint32_t*>(nib + q * 1024 + ((2 + g_lo) * 16 + nn) * nb * 4 + j * 4);
-    const float scale = e8m0(scl[q * 64 + nn * 4 + j]);
-    const float w0 = bf16r(kE2M1[(d0 >> shift) & 15u] * scale);
-    const float w1 = bf16r(kE2M1[(d1 >> shift) & 15u] * scale);
-#pragma unroll
-    for (int t = 0; t < kChunkMax; ++t) {
-      if (t < count) {
-        const uint16_t* xr = s_in[t] + b * kBlock;
-        acc[t] = acc[t] + w0 * bf16_to_f32(xr[l]);
-        acc[t] = acc[t] + w1 * bf16_to_f32(xr[l + 16]);
-      }
-    }
-  }
-  __shared__ float s_lane[kTileRows][16][kChunkMax + 1];
-  __shared__ float s_gu[kTileRows][kChunkMax];
-#pragma unroll
-  for (int t = 0; t < kChunkMax; ++t)
-    if (t < count) s_lane[nn][l][t] = acc[t];
-  __syncthreads();
-  for (int t = l; t < count; t += 16) {
-    float sum = -0.0f;
-    for (int ll = 0; ll < 16; ++ll) sum = sum + s_lane[nn][ll][t];
-    const float bias = (a.bias != nullptr && n < rows) ? a.bias[(size_t)expert * a.bias_expert_stride + n] : 0.0f;
-    const float total = bias + sum;
-    const int slot = a.route_slot[start + t];
-    if (MODE == kDown) {
-      if (n < rows) a.y[(size_t)slot * rows + n] = bf16_bits(total);  // bf16 (cpu_runner.rs:2945-2947)
-    } else {
-      const float gu = bf16r(total);  // bf16 (cpu_runner.rs:2905)
-      s_gu[nn][t] = gu;
-      if (a.trace_gu != nullptr && n < rows) a.trace_gu[(size_t)slot * rows + n] = gu;
-    }
-  }
-  if (MODE == kGateUp) {
-    __syncthreads();
-    const int half = rows / 2;
-    for (int idx = tid; idx < (kTileRows / 2) * count; idx += blockDim.x) {
-      const int p = idx % (kTileRows / 2), t = idx / (kTileRows / 2);
-      const int i = tile * (kTileRows / 2) + p;
-      if (i < half) {
-        const float act = swiglu_one(s_gu[2 * p][t], s_gu[2 * p + 1][t], a.alpha, a.limit, a.sig_tab);
-        a.act_next16[(size_t)(start + t) * half + i] = bf16_bits(act);  // activated_bf16 (cpu_runner.rs:2917)
-        if (a.trace_sw != nullptr) a.trace_sw[(size_t)a.route_slot[start + t] * half + i] = act;
-      }
-    }
+  for (int t0 = 0; t0 < rec.z; t0 += routes) {  // uniform
+    const int count = min(routes, rec.z - t0);
+    float* fold = reinterpret_cast<float*>(s_exact);
+    if (count <= 1) exact_pass<MODE, 1>(a, rec.x, rec.y + t0, count, s_exact, fold);
+    else if (count <= 4) exact_pass<MODE, 4>(a, rec.x, rec.y + t0, count, s_exact, fold);
+    else exact_pass<MODE, kExactRoutes>(a, rec.x, rec.y + t0, count, s_exact, fold);
   }
 }
 
@@ -3982,9 +4110,14 @@ hipError_t launch_down_combine(const GemmArgs& d, const float* weights, int top_
 }
 
 hipError_t launch_exact(GemmMode mode, const GemmArgs& a, int grid_work, hipStream_t stream) {
-  const dim3 grid((unsigned)a.w.tiles, (unsigned)grid_work);
-  if (mode == kGateUp) hipLaunchKernelGGL(exact_kernel<kGateUp>, grid, dim3(256), 0, stream, a);
-  else if (mode == kDown) hipLaunchKernelGGL(exact_kernel<kDown>, grid, dim3(256), 0, stream, a);
+  const dim3 grid((unsigned)((a.w.rows + kExactRows - 1) / kExactRows), (unsigned)grid_work);
+  // Routes per pass: 8, or as many as the LDS holds (K > 10,000 or so).
+  const size_t K = a.w.blocks * kBlock, limit = 160 * 1024 - 1024;
+  const int routes = exact_lds(K, kExactRoutes) <= limit ? kExactRoutes : exact_lds(K, 4) <= limit ? 4 : 1;
+  const unsigned lds = (unsigned)exact_lds(K, routes);
+  if (lds > limit) return hipErrorInvalidValue;
+  if (mode == kGateUp) hipLaunchKernelGGL(exact_kernel<kGateUp>, grid, dim3(256), lds, stream, a, routes);
+  else if (mode == kDown) hipLaunchKernelGGL(exact_kernel<kDown>, grid, dim3(256), lds, stream, a, routes);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }

@@ -122,6 +122,28 @@ def test_exact_bf16_sums_in_sixteen_ordered_lanes(ctx):
     close(layer)
 
 
+@pytest.mark.parametrize("m,shrink,scales", [(1, 0, False), (9, 0, True), (37, 64, False), (40, 0, False), (70, 64, True)])
+def test_exact_bf16_passes_and_inexact_products(ctx, m, shrink, scales):
+    """exact_kernel's passes of 1, 4 and 8 routes (all 1..8 remainders occur),
+    a partial last K group and last row tile, inputs of about 2^-64 and scale
+    bytes at both ends of E8M0 (products that round before they are added)."""
+    host = O.synthetic_layer(43, 0, experts=5, hidden=160, intermediate=96, top_k=3)
+    x = O.gen_hidden(43, 700 + m, m, 160)
+    logits = O.bf16_round_array(np.random.default_rng(m).standard_normal((m, 5)).astype(np.float32))
+    if shrink:
+        x = synth.bf16_bits(synth.bf16_to_f32(x) * np.float32(2.0 ** -shrink))
+    if scales:
+        records = host.gate_up.reshape(-1, 17)
+        records[::7, 0] = np.resize(np.array([0, 1, 2, 100, 140, 180], np.uint8), records[::7].shape[0])
+    want = O.moe_batch(host, x, injected_logits=logits, trace=True, projection=G.PROJECTION_EXACT_BF16)
+    assert want["status"] == O.OK
+    layer = gpu_layer(ctx, host, G.PROJECTION_EXACT_BF16)
+    got = layer.forward(x, injected_logits=logits, trace=True)
+    assert_moe_equal(got, want)
+    assert_traces_equal(got, want)
+    close(layer)
+
+
 def test_unknown_projection_is_rejected(ctx):
     host = O.synthetic_layer(3, 0, experts=2, hidden=64, intermediate=32, top_k=1)
     with pytest.raises(G.GossmxError) as e:
