@@ -1,43 +1,46 @@
 // The dense path around the MoE block: the rest of a GPT-OSS decoder step as
 // CpuModel::prepare_step runs it (crates/gpt-oss-model-runner/src/
-// cpu_runner.rs:2103-2333, forward_layer_batch :2335-2586). Norms, RoPE,
-// attention and the KV cache run on the host; the projections and each
-// layer's MoE half (post-attention RMSNorm, moe_batch, residual add, through
-// gossmx_moe_forward_residual) on the GPU.
+// cpu_runner.rs:2103-2333, forward_layer_batch :2335-2586), on the GPU: a step
+// is one copy in (the embedding rows), launches on the context's stream, one
+// copy out (the logits) and one synchronization. Each layer's MoE half
+// (post-attention RMSNorm, moe_batch, residual add) goes through
+// gossmx_moe_forward_residual. The steps used to run norms, RoPE and attention
+// on host threads with two round trips a layer: a 63-token prefill and 8
+// decodes of two GPT-OSS-20B layers went from 9.76 to 4.67 ms.
 //
 // - bf16 projections: Kernels::bf16_matvec (gpt-oss-cpu-kernels lib.rs:314-341)
 //   with its 16 fixed reduction lanes, multiply then add, lanes folded 0..15
 //   (scalar_bf16_dot lib.rs:1007-1029), then += bias (project_bf16[_batch]
-//   cpu_runner.rs:2689-2792): dense_proj_kernel, over copies of the Q/K/V/O
-//   weights and lm_head made in HBM when the model is created.
+//   cpu_runner.rs:2689-2792): dense_proj_kernel and dense_gemv_kernel, over
+//   copies of the Q/K/V/O weights and lm_head made in HBM when the model is
+//   created.
 // - RMSNorm boundaries: norm_boundary (:2680-2687) over Kernels::rms_norm
-//   (lib.rs:699-730, the same 16-lane sum of squares).
-// - YaRN RoPE (YarnRope :3927-4013) with its bf16 boundaries.
+//   (lib.rs:699-730, the same 16-lane sum of squares): dense_norm_kernel.
+// - YaRN RoPE (YarnRope :3927-4013) with its bf16 boundaries, by the host's
+//   cosines and sines: qkv_finish_kernel.
 // - Attention with learned sinks over the visible KV window
-//   (attention_one_staged :3840-3924), and the KV cache of CpuKvCache
-//   (:653-740): a sliding layer keeps sliding_window tokens, a full layer
-//   context_cap. A step's rows are staged and committed to the caches only
-//   when the whole step succeeded (PreparedCpuStep::commit, :1081-1113).
+//   (attention_one_staged :3840-3924): attention_kernel. The KV cache of
+//   CpuKvCache (:653-740): a sliding layer keeps sliding_window tokens, a full
+//   layer context_cap. A step's rows count as cached only when the whole step
+//   succeeded (PreparedCpuStep::commit, :1081-1113).
 // - Residual adds (add_residual :3732-3738), the final norm, lm_head and its
 //   bf16 round trip with the finiteness check (:2255-2312).
-// expf, powf, cosf, sinf and log are the host C library's: the functions
-// Rust's f32/f64 methods call on x86_64 Linux.
+// powf, cosf, sinf and log are the host C library's, as is expf in
+// gossmx_attention: the functions Rust's f32/f64 methods call on x86_64 Linux
+// (attention_kernel's expf_glibc has the same results).
 
 #include "../../include/gossmx.h"
 #include "gossmx_internal.h"
 
 #include <algorithm>
-#include <atomic>
 #include <chrono>
 #include <cmath>
-#include <condition_variable>
 #include <cstdio>
 #include <cstring>
-#include <functional>
 #include <memory>
-#include <mutex>
 #include <new>
-#include <thread>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 namespace {
@@ -56,91 +59,6 @@ inline uint16_t bf16_bits(float f) {
 }
 inline float bf16_f32(uint16_t b) { return u2f((uint32_t)b << 16); }
 inline float bf16_round(float f) { return bf16_f32(bf16_bits(f)); }
-
-// ---------------------------------------------------------------------------
-// Worker pool: run(n, fn) calls fn(i) for every i < n on the pool's threads
-// and the caller's, and returns when all calls have returned.
-
-class Pool {
- public:
-  explicit Pool(size_t threads) {
-    for (size_t i = 1; i < threads; ++i) workers_.emplace_back([this] { loop(); });
-  }
-  ~Pool() {
-    {
-      std::lock_guard<std::mutex> g(m_);
-      stop_ = true;
-      ++generation_;
-    }
-    wake_.notify_all();
-    for (auto& t : workers_) t.join();
-  }
-  size_t size() const { return workers_.size() + 1; }
-  void run(size_t n, const std::function<void(size_t)>& fn) {
-    if (workers_.empty() || n <= 1) {
-      for (size_t i = 0; i < n; ++i) fn(i);
-      return;
-    }
-    {
-      std::lock_guard<std::mutex> g(m_);
-      fn_ = &fn;
-      n_ = n;
-      next_.store(0);
-      pending_ = workers_.size();
-      ++generation_;
-    }
-    wake_.notify_all();
-    work();
-    std::unique_lock<std::mutex> l(m_);
-    done_.wait(l, [this] { return pending_ == 0; });
-  }
-
- private:
-  void work() {
-    for (size_t i; (i = next_.fetch_add(1)) < n_;) (*fn_)(i);
-  }
-  void loop() {
-    uint64_t seen = 0;
-    for (;;) {
-      {
-        std::unique_lock<std::mutex> l(m_);
-        wake_.wait(l, [&] { return generation_ != seen; });
-        seen = generation_;
-        if (stop_) return;
-      }
-      work();
-      std::lock_guard<std::mutex> g(m_);
-      if (--pending_ == 0) done_.notify_one();
-    }
-  }
-  std::vector<std::thread> workers_;
-  std::mutex m_;
-  std::condition_variable wake_, done_;
-  const std::function<void(size_t)>* fn_ = nullptr;
-  size_t n_ = 0, pending_ = 0;
-  std::atomic<size_t> next_{0};
-  uint64_t generation_ = 0;
-  bool stop_ = false;
-};
-
-// norm_boundary: bf16 -> f32, rms_norm, -> bf16.
-void norm_boundary(const uint16_t* x, const float* w, size_t n, float eps, uint16_t* out) {
-  float lanes[16] = {0};
-  size_t i = 0;
-  for (; i + 16 <= n; i += 16)
-    for (int l = 0; l < 16; ++l) {
-      const float v = bf16_f32(x[i + l]);
-      lanes[l] += v * v;
-    }
-  for (size_t l = 0; i < n; ++i, ++l) {
-    const float v = bf16_f32(x[i]);
-    lanes[l] += v * v;
-  }
-  float ss = 0.0f;
-  for (int l = 0; l < 16; ++l) ss += lanes[l];
-  const float inv = 1.0f / std::sqrt(ss / (float)n + eps);
-  for (size_t k = 0; k < n; ++k) out[k] = bf16_bits(bf16_f32(x[k]) * inv * w[k]);
-}
 
 // ---------------------------------------------------------------------------
 // YaRN RoPE (YarnRope::new / apply, cpu_runner.rs:3933-4013).
@@ -185,17 +103,21 @@ Rope make_rope(const gossmx_model_config& c) {
   return r;
 }
 
-// The bf16 cosine and sine of a position depend on (position, i) only: they
-// are computed once per call and shared by every head.
-void rope_apply(const Rope& r, float* v, size_t heads, size_t position) {
+// The bf16 cosines, then sines, of a position: they depend on (position, i)
+// only and every head shares them.
+void rope_row(const Rope& r, size_t position, float* table) {
   const size_t half = r.head_dim / 2;
-  thread_local std::vector<float> table;
-  table.resize(2 * half);
   for (size_t i = 0; i < half; ++i) {
     const float angle = (float)position * r.inv_freq[i];
     table[i] = bf16_round(cosf(angle) * r.attention_scale);
     table[half + i] = bf16_round(sinf(angle) * r.attention_scale);
   }
+}
+
+void rope_apply(const Rope& r, float* v, size_t heads, size_t position) {
+  const size_t half = r.head_dim / 2;
+  std::vector<float> table(2 * half);
+  rope_row(r, position, table.data());
   for (size_t h = 0; h < heads; ++h) {
     float* p = v + h * r.head_dim;
     for (size_t i = 0; i < half; ++i) {
@@ -213,21 +135,21 @@ void rope_apply(const Rope& r, float* v, size_t heads, size_t position) {
 // Attention for one query over `tokens` visible key/value rows, oldest first
 // (attention_one_staged): bf16 QK dot, bf16 scale, softmax with the sink in
 // the denominator, bf16 probabilities, f32 accumulation, bf16 output.
-// key(t) / value(t) return the row of visible token t (all kv heads). Heads
-// are independent: this computes heads [h_begin, h_end) of out.
+// keys and values are rows of kv_heads * head_dim. gossmx_attention's; a
+// model's steps run attention_kernel, with the same float chains.
 
-template <class KeyRow, class ValueRow>
-void attention(const float* q_all, size_t tokens, const KeyRow& key, const ValueRow& value, const float* sinks,
-               size_t heads, size_t kv_heads, size_t head_dim, float* out, std::vector<float>& scores,
-               size_t h_begin, size_t h_end) {
-  const size_t groups = heads / kv_heads;
-  const float scale = 1.0f / std::sqrt((float)head_dim);
-  scores.resize(tokens);
-  for (size_t h = h_begin; h < h_end; ++h) {
+float attention_scale(size_t head_dim) { return 1.0f / std::sqrt((float)head_dim); }
+
+void attention(const float* q_all, size_t tokens, const uint16_t* keys, const uint16_t* values, const float* sinks,
+               size_t heads, size_t kv_heads, size_t head_dim, float* out) {
+  const size_t groups = heads / kv_heads, width = kv_heads * head_dim;
+  const float scale = attention_scale(head_dim);
+  std::vector<float> scores(tokens);
+  for (size_t h = 0; h < heads; ++h) {
     const float* q = q_all + h * head_dim;
     const size_t kvh = h / groups;
     for (size_t t = 0; t < tokens; ++t) {
-      const uint16_t* k = key(t) + kvh * head_dim;
+      const uint16_t* k = keys + t * width + kvh * head_dim;
       float dot = 0.0f;
       for (size_t d = 0; d < head_dim; ++d) dot += q[d] * bf16_f32(k[d]);
       dot = bf16_round(dot);
@@ -242,28 +164,23 @@ void attention(const float* q_all, size_t tokens, const KeyRow& key, const Value
     for (size_t d = 0; d < head_dim; ++d) o[d] = 0.0f;
     for (size_t t = 0; t < tokens; ++t) {
       const float p = bf16_round(expf(scores[t] - maximum) / denominator);
-      const uint16_t* v = value(t) + kvh * head_dim;
+      const uint16_t* v = values + t * width + kvh * head_dim;
       for (size_t d = 0; d < head_dim; ++d) o[d] += p * bf16_f32(v[d]);
     }
     for (size_t d = 0; d < head_dim; ++d) o[d] = bf16_round(o[d]);
   }
 }
 
-// Committed KV rows of one layer (CpuKvCache): the last min(positions, capacity)
-// tokens, position p in slot p % capacity.
+// The KV cache of one layer (CpuKvCache): the last min(positions, capacity)
+// tokens are committed. On the device it is a ring of `slots` rows, position p
+// in slot p % slots, with room for the m rows of a step beside every committed
+// row that a later step can still see (the last capacity - 1): a step writes
+// its rows there, and committing them is the host's `len` and `start` alone.
 struct KvCache {
-  size_t capacity = 0, width = 0, len = 0, start = 0;
-  std::vector<uint16_t> k, v;
-  const uint16_t* key(size_t p) const { return k.data() + (p % capacity) * width; }
-  const uint16_t* value(size_t p) const { return v.data() + (p % capacity) * width; }
-  void append(size_t p, const uint16_t* key_row, const uint16_t* value_row) {
-    const size_t slots = std::min(p + 1, capacity);
-    if (k.size() < slots * width) {
-      k.resize(std::min(capacity, std::max(slots, 2 * k.size() / std::max<size_t>(width, 1))) * width);
-      v.resize(k.size());
-    }
-    std::memcpy(k.data() + (p % capacity) * width, key_row, width * 2);
-    std::memcpy(v.data() + (p % capacity) * width, value_row, width * 2);
+  size_t capacity = 0, len = 0, start = 0;
+  size_t slots = 0;
+  uint16_t *k = nullptr, *v = nullptr;
+  void append(size_t p) {
     if (len == capacity) ++start;
     else ++len;
     if (len == 1) start = p;
@@ -287,34 +204,31 @@ int check_config(const gossmx_model_config* c) {
 
 }  // namespace
 
-// The model's device side: the projection weights and lm_head copied to HBM,
-// and grow-only f32 staging for the projections' inputs and outputs (device
-// buffers, and pinned host buffers for the copies).
+// The model's device side: its dense tensors but the embedding copied to HBM,
+// the RoPE table, and grow-only buffers for a step's rows.
 struct DenseDevice {
   struct Layer {
     const uint16_t *q, *k, *v, *o;
     const float *qb, *kb, *vb, *ob;
-    const float* post_norm;  // post_attention_norm, for the MoE call in device memory
+    const float *input_norm, *post_norm, *sinks;
   };
   int device = 0;
   std::vector<void*> weights;  // device allocations of the copies
   std::vector<Layer> layers;
   const uint16_t* lm_head = nullptr;
-  float *d_in = nullptr, *d_out = nullptr, *h_in = nullptr, *h_out = nullptr;
-  size_t in_cap = 0, out_cap = 0;  // floats
-  // The residual rows around the MoE call: device hidden, after and next
-  // (m x hidden bf16 each) and their pinned staging, as floats' worth of bytes.
-  float *d_rows = nullptr, *h_rows = nullptr;
-  size_t rows_cap = 0;
+  const float* final_norm = nullptr;
+  float* rope = nullptr;  // cosines and sines (rope_row) of the positions below rope_rows
+  size_t rope_rows = 0;
+  char *work = nullptr, *host_in = nullptr, *host_out = nullptr;  // a step's device rows; pinned input and results
+  size_t work_cap = 0, in_cap = 0, out_cap = 0;                  // bytes
+  double clock_hz = 1e8;  // of wall_clock64
   ~DenseDevice() {
     (void)hipSetDevice(device);
     for (void* p : weights) (void)hipFree(p);
-    (void)hipFree(d_in);
-    (void)hipFree(d_out);
-    (void)hipFree(d_rows);
-    (void)hipHostFree(h_in);
-    (void)hipHostFree(h_out);
-    (void)hipHostFree(h_rows);
+    (void)hipFree(rope);
+    (void)hipFree(work);
+    (void)hipHostFree(host_in);
+    (void)hipHostFree(host_out);
   }
 };
 
@@ -322,15 +236,19 @@ struct gossmx_model {
   gossmx_ctx* ctx = nullptr;
   gossmx_model_config cfg{};
   const uint16_t* embedding = nullptr;
-  const float* final_norm = nullptr;
-  const uint16_t* lm_head = nullptr;
   std::vector<gossmx_dense_layer> layers;
   Rope rope;
   std::vector<KvCache> caches;
   size_t position = 0;
-  std::unique_ptr<Pool> pool;
   DenseDevice dev;
   double dense_seconds = 0.0, moe_seconds = 0.0;
+  ~gossmx_model() {
+    (void)hipSetDevice(dev.device);
+    for (KvCache& kv : caches) {
+      (void)hipFree(kv.k);
+      (void)hipFree(kv.v);
+    }
+  }
 };
 
 namespace {
@@ -359,244 +277,268 @@ int upload(DenseDevice& D, const T* src, size_t n, const T** dst) {
   return GOSSMX_OK;
 }
 
-int grow(float** dev, float** host, size_t* cap, size_t n) {
+// Grows a device (or, pinned, a host) buffer to n bytes; its contents go.
+int grow(char** p, size_t* cap, size_t n, bool pinned) {
   if (n <= *cap) return GOSSMX_OK;
-  (void)hipFree(*dev);
-  (void)hipHostFree(*host);
-  *dev = *host = nullptr;
+  if (pinned) (void)hipHostFree(*p);
+  else (void)hipFree(*p);
+  *p = nullptr;
   *cap = 0;
-  DENSE_HIP(hipMalloc(dev, n * sizeof(float)), "projection buffer");
-  DENSE_HIP(hipHostMalloc(host, n * sizeof(float)), "projection staging");
+  if (pinned) DENSE_HIP(hipHostMalloc((void**)p, n), "step staging");
+  else DENSE_HIP(hipMalloc((void**)p, n), "step buffer");
   *cap = n;
   return GOSSMX_OK;
 }
 
-// One projection of the rows `in` (m x cols bf16) by w ([rows][cols] bf16 in
-// HBM) + bias, into out (m x rows f32, host).
-struct Projection {
-  const uint16_t* w;
-  const float* bias;
-  size_t rows;
-  float* out;
-};
-
-// Runs the projections of one input on the GPU (project_bf16_batch): one copy
-// in, one launch each, one copy out, one synchronization.
-int gpu_project_impl(gossmx_model* M, const uint16_t* in, size_t m, size_t cols, const Projection* p,
-                     size_t count) {
+// The RoPE table covers positions below `rows`. It doubles, so a sequence
+// computes each position's cosines and sines (host cosf and sinf) about twice
+// at most.
+int grow_rope(gossmx_model* M, size_t rows, hipStream_t stream) {
   DenseDevice& D = M->dev;
-  // The context's stream is read on every call: gossmx_ctx_set_stream may
-  // have replaced it since the model was created.
-  const hipStream_t stream = gossmx::context_stream(M->ctx);
-  size_t total = 0;
-  for (size_t i = 0; i < count; ++i) total += m * p[i].rows;
-  DENSE_HIP(hipSetDevice(D.device), "hipSetDevice");
-  if (int st = grow(&D.d_in, &D.h_in, &D.in_cap, m * cols)) return st;
-  if (int st = grow(&D.d_out, &D.h_out, &D.out_cap, total)) return st;
-  for (size_t i = 0; i < m * cols; ++i) D.h_in[i] = bf16_f32(in[i]);
-  gossmx::count_transfer(gossmx::kTransferActivation, m * cols * sizeof(float));
-  DENSE_HIP(hipMemcpyAsync(D.d_in, D.h_in, m * cols * sizeof(float), hipMemcpyHostToDevice, stream),
-            "projection input copy");
-  // One launch per group. One token through small matrices (Q/K/V, O):
-  // work-groups stage their whole K range at once; lm_head and batches: the
-  // K-chunked kernel.
-  if (count > 3) return err(GOSSMX_ERR_INVALID_ARGUMENT, "internal: more than three projections in a group");
-  gossmx::DenseSet set{};
-  size_t off = 0;
-  for (size_t i = 0; i < count; ++i) {
-    set.w[i] = p[i].w;
-    set.bias[i] = p[i].bias;
-    set.out[i] = D.d_out + off;
-    set.rows[i] = (int)p[i].rows;
-    off += m * p[i].rows;
+  if (rows <= D.rope_rows) return GOSSMX_OK;
+  const size_t dim = M->cfg.head_dim;
+  const size_t n = std::max(rows, std::min(std::max<size_t>(2 * D.rope_rows, 64), M->cfg.context_cap));
+  std::vector<float> table(n * dim);
+  for (size_t p = 0; p < n; ++p) rope_row(M->rope, p, &table[p * dim]);
+  float* d = nullptr;
+  DENSE_HIP(hipMalloc((void**)&d, n * dim * sizeof(float)), "rotation table");
+  gossmx::count_transfer(gossmx::kTransferUpload, n * dim * sizeof(float));
+  hipError_t e = hipMemcpyAsync(d, table.data(), n * dim * sizeof(float), hipMemcpyHostToDevice, stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(stream);
+  if (e != hipSuccess) {
+    (void)hipFree(d);
+    return hip_err(e, "rotation table copy");
   }
-  const bool whole_k = m == 1 && cols % 8 == 0 && cols <= 4096 && total <= 65536;
-  DENSE_HIP(whole_k ? gossmx::launch_dense_gemv(set, (int)count, D.d_in, (int)cols, stream)
-                    : gossmx::launch_dense_proj(set, (int)count, D.d_in, (int)cols, (int)m, stream),
-            "projection launch");
-  gossmx::count_transfer(gossmx::kTransferOutput, total * sizeof(float));
-  DENSE_HIP(hipMemcpyAsync(D.h_out, D.d_out, total * sizeof(float), hipMemcpyDeviceToHost, stream),
-            "projection output copy");
-  DENSE_HIP(hipStreamSynchronize(stream), "projection");
-  off = 0;
-  for (size_t i = 0; i < count; ++i) {
-    std::memcpy(p[i].out, D.h_out + off, m * p[i].rows * sizeof(float));
-    off += m * p[i].rows;
-  }
+  (void)hipFree(D.rope);
+  D.rope = d;
+  D.rope_rows = n;
   return GOSSMX_OK;
 }
 
-// A run-time failure of the round trip (HIP error, out of memory) opens the
-// circuit breaker, as a failed projection call does.
-int gpu_project(gossmx_model* M, const uint16_t* in, size_t m, size_t cols, const Projection* p, size_t count) {
-  return gossmx::run_time_result(M->ctx, gpu_project_impl(M, in, m, cols, p, count));
+// Room for m rows at position `base` in a layer's ring (KvCache). A larger
+// ring takes the committed rows that can still be seen to their new slots.
+int grow_ring(gossmx_model* M, KvCache& kv, size_t base, size_t m, hipStream_t stream) {
+  const size_t needed = std::min(base, kv.capacity - 1) + m;
+  if (needed <= kv.slots) return GOSSMX_OK;
+  const size_t width = M->cfg.kv_heads * M->cfg.head_dim;
+  const size_t n = std::max(needed, std::min(std::max<size_t>(2 * kv.slots, 256), M->cfg.context_cap));
+  uint16_t* ring[2] = {nullptr, nullptr};
+  hipError_t e = hipMalloc((void**)&ring[0], n * width * 2);
+  if (e == hipSuccess) e = hipMalloc((void**)&ring[1], n * width * 2);
+  const size_t keep = std::min(kv.len, kv.capacity - 1);
+  for (size_t p = base - keep; p < base && e == hipSuccess;) {
+    const size_t from = p % kv.slots, to = p % n, run = std::min(base - p, std::min(kv.slots - from, n - to));
+    for (int i = 0; i < 2 && e == hipSuccess; ++i)
+      e = hipMemcpyAsync(ring[i] + to * width, (i ? kv.v : kv.k) + from * width, run * width * 2,
+                         hipMemcpyDeviceToDevice, stream);
+    p += run;
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(stream);
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(stream);
+    (void)hipFree(ring[0]);
+    (void)hipFree(ring[1]);
+    return hip_err(e, "KV cache growth");
+  }
+  (void)hipFree(kv.k);
+  (void)hipFree(kv.v);
+  kv.k = ring[0];
+  kv.v = ring[1];
+  kv.slots = n;
+  return GOSSMX_OK;
 }
 
-// The rest of a layer after attention, in one round trip: the O projection of
-// attn (m x QW bf16), the residual add with hidden, and the MoE half
-// (post-attention norm, block, residual add) in device memory; hidden
-// (m x H bf16) becomes the next layer's rows. The MoE time is added to *moe.
-int gpu_o_residual_moe_impl(gossmx_model* M, const gossmx_dense_layer& L, const DenseDevice::Layer& DL,
-                            const uint16_t* attn, size_t m, uint16_t* hidden, double* moe) {
+// Up to three projections of one input (project_bf16[_batch]) in one launch.
+// One token through small matrices (Q/K/V, O): work-groups stage their whole K
+// range at once; batches: the K-chunked kernel.
+hipError_t project(const gossmx::DenseSet& set, int count, const float* in, size_t cols, size_t m, hipStream_t stream) {
+  size_t rows = 0;
+  for (int i = 0; i < count; ++i) rows += set.rows[i];
+  return m == 1 && cols % 8 == 0 && cols <= 4096 && rows <= 65536
+             ? gossmx::launch_dense_gemv(set, count, in, (int)cols, stream)
+             : gossmx::launch_dense_proj(set, count, in, (int)cols, (int)m, stream);
+}
+
+// A step's buffers in DenseDevice::work: m rows each.
+struct StepRows {
+  uint16_t *hidden, *after, *next;      // [hidden] bf16
+  float *x, *q, *k, *v, *proj;          // the next projections' input; Q, K, V and O outputs
+  char* out;                            // the results that go to the host: marks, logits
+};
+
+size_t out_bytes(const gossmx_model_config& c) { return c.layers * sizeof(gossmx::ModelMark) + c.vocab * 2; }
+
+// Enqueues one layer-major step over the m rows whose embeddings are in
+// host_in, and the copy of its marks and the last row's logits to host_out.
+int enqueue_step(gossmx_model* M, size_t m, const StepRows& R, hipStream_t stream) {
+  const gossmx_model_config& c = M->cfg;
   DenseDevice& D = M->dev;
-  const hipStream_t stream = gossmx::context_stream(M->ctx);
-  const size_t H = M->cfg.hidden, QW = M->cfg.heads * M->cfg.head_dim, n = m * H;
-  DENSE_HIP(hipSetDevice(D.device), "hipSetDevice");
-  if (int st = grow(&D.d_in, &D.h_in, &D.in_cap, m * QW)) return st;
-  if (int st = grow(&D.d_out, &D.h_out, &D.out_cap, n)) return st;
-  if (int st = grow(&D.d_rows, &D.h_rows, &D.rows_cap, (3 * n + 1) / 2)) return st;
-  uint16_t* d_hidden = reinterpret_cast<uint16_t*>(D.d_rows);
-  uint16_t *d_after = d_hidden + n, *d_next = d_hidden + 2 * n;
-  uint16_t* h_rows = reinterpret_cast<uint16_t*>(D.h_rows);
-  for (size_t i = 0; i < m * QW; ++i) D.h_in[i] = bf16_f32(attn[i]);
-  std::memcpy(h_rows, hidden, n * 2);
-  gossmx::count_transfer(gossmx::kTransferActivation, m * QW * sizeof(float) + n * 2);
-  DENSE_HIP(hipMemcpyAsync(D.d_in, D.h_in, m * QW * sizeof(float), hipMemcpyHostToDevice, stream),
-            "projection input copy");
-  DENSE_HIP(hipMemcpyAsync(d_hidden, h_rows, n * 2, hipMemcpyHostToDevice, stream), "residual rows copy");
-  gossmx::DenseSet set{};
-  set.w[0] = DL.o;
-  set.bias[0] = DL.ob;
-  set.out[0] = D.d_out;
-  set.rows[0] = (int)H;
-  const bool whole_k = m == 1 && QW % 8 == 0 && QW <= 4096;
-  DENSE_HIP(whole_k ? gossmx::launch_dense_gemv(set, 1, D.d_in, (int)QW, stream)
-                    : gossmx::launch_dense_proj(set, 1, D.d_in, (int)QW, (int)m, stream),
-            "projection launch");
-  DENSE_HIP(gossmx::launch_residual_add(d_hidden, D.d_out, d_after, n, stream), "residual add launch");
-  const auto t_moe = std::chrono::steady_clock::now();
-  gossmx_moe_io io{};
-  io.x = d_after;
-  io.m = m;
-  io.memory = GOSSMX_MEM_DEVICE;
-  int st = gossmx_moe_forward_residual(M->ctx, L.moe, &io, DL.post_norm, M->cfg.rms_norm_eps, d_next);
-  (void)gossmx_profile_tag(M->ctx, -1, GOSSMX_PHASE_UNKNOWN);
-  if (st == GOSSMX_OK) {
-    // gossmx_synchronize reports the device error flags.
-    gossmx::count_transfer(gossmx::kTransferOutput, n * 2);
-    const hipError_t e = hipMemcpyAsync(h_rows + n, d_next, n * 2, hipMemcpyDeviceToHost, stream);
-    st = e == hipSuccess ? gossmx_synchronize(M->ctx) : hip_err(e, "next rows copy");
+  const size_t H = c.hidden, QW = c.heads * c.head_dim, KW = c.kv_heads * c.head_dim, n = m * H;
+  const size_t base = M->position;
+  gossmx::ModelMark* marks = reinterpret_cast<gossmx::ModelMark*>(R.out);
+  uint16_t* logits = reinterpret_cast<uint16_t*>(R.out + c.layers * sizeof(gossmx::ModelMark));
+  const int* flags = gossmx::context_error_flags(M->ctx);
+  gossmx::count_transfer(gossmx::kTransferActivation, n * 2);
+  DENSE_HIP(hipMemcpyAsync(R.hidden, D.host_in, n * 2, hipMemcpyHostToDevice, stream), "embedding rows copy");
+  uint16_t *hidden = R.hidden, *next = R.next;
+  for (size_t li = 0; li < c.layers; ++li) {
+    const DenseDevice::Layer& L = D.layers[li];
+    KvCache& kv = M->caches[li];
+    DENSE_HIP(gossmx::launch_dense_norm(hidden, L.input_norm, (int)m, (int)H, c.rms_norm_eps, R.x,
+                                        li ? marks + li - 1 : nullptr, flags, stream),
+              "input norm launch");
+    gossmx::DenseSet qkv{};
+    const uint16_t* w[3] = {L.q, L.k, L.v};
+    const float* bias[3] = {L.qb, L.kb, L.vb};
+    float* out[3] = {R.q, R.k, R.v};
+    for (int i = 0; i < 3; ++i) {
+      qkv.w[i] = w[i];
+      qkv.bias[i] = bias[i];
+      qkv.out[i] = out[i];
+      qkv.rows[i] = (int)(i ? KW : QW);
+    }
+    DENSE_HIP(project(qkv, 3, R.x, H, m, stream), "projection launch");
+    gossmx::AttnArgs a{};
+    a.q = R.q;
+    a.k_new = R.k;
+    a.v_new = R.v;
+    a.rope = D.rope;
+    a.k = kv.k;
+    a.v = kv.v;
+    a.sinks = L.sinks;
+    a.out = R.x;
+    a.base = base;
+    a.len = kv.len;
+    a.capacity = kv.capacity;
+    a.slots = kv.slots;
+    a.m = (int)m;
+    a.heads = (int)c.heads;
+    a.kv_heads = (int)c.kv_heads;
+    a.head_dim = (int)c.head_dim;
+    a.scale = attention_scale(c.head_dim);
+    DENSE_HIP(gossmx::launch_attention(a, stream), "attention launch");
+    gossmx::DenseSet o{};
+    o.w[0] = L.o;
+    o.bias[0] = L.ob;
+    o.out[0] = R.proj;
+    o.rows[0] = (int)H;
+    DENSE_HIP(project(o, 1, R.x, QW, m, stream), "projection launch");
+    DENSE_HIP(gossmx::launch_residual_add(hidden, R.proj, R.after, n, &marks[li].begin, stream), "residual add launch");
+    // The MoE half (norm_boundary(after, post_attention_norm), moe_batch,
+    // add_residual) -> the next layer's rows. The block's profile records carry
+    // the layer and the phase.
+    (void)gossmx_profile_tag(M->ctx, (int)li, base == 0 || m > 1 ? GOSSMX_PHASE_PREFILL : GOSSMX_PHASE_DECODE);
+    gossmx_moe_io io{};
+    io.x = R.after;
+    io.m = m;
+    io.memory = GOSSMX_MEM_DEVICE;
+    const int st = gossmx_moe_forward_residual(M->ctx, M->layers[li].moe, &io, L.post_norm, c.rms_norm_eps, next);
+    (void)gossmx_profile_tag(M->ctx, -1, GOSSMX_PHASE_UNKNOWN);
+    if (st != GOSSMX_OK) return st;
+    std::swap(hidden, next);
   }
-  *moe += seconds_since(t_moe);
+  // Final norm and lm_head for the last row (the only row whose logits are required).
+  DENSE_HIP(gossmx::launch_dense_norm(hidden + (m - 1) * H, D.final_norm, 1, (int)H, c.rms_norm_eps, R.x,
+                                      marks + c.layers - 1, flags, stream),
+            "final norm launch");
+  DENSE_HIP(gossmx::launch_lm_head(D.lm_head, R.x, logits, (int)c.vocab, (int)H, stream), "projection launch");
+  gossmx::count_transfer(gossmx::kTransferOutput, out_bytes(c));
+  DENSE_HIP(hipMemcpyAsync(D.host_out, R.out, out_bytes(c), hipMemcpyDeviceToHost, stream), "logits copy");
+  return GOSSMX_OK;
+}
+
+// The GPU side of a step: one copy in, its launches, one copy out, one
+// synchronization. The MoE calls' error flags are reported as the first layer
+// that raised any left them; *moe becomes the time between the marks.
+int gpu_step(gossmx_model* M, const uint32_t* tokens, size_t m, double* moe) {
+  const gossmx_model_config& c = M->cfg;
+  DenseDevice& D = M->dev;
+  // The context's stream is read on every step: gossmx_ctx_set_stream may have
+  // replaced it since the last one.
+  const hipStream_t stream = gossmx::context_stream(M->ctx);
+  const size_t H = c.hidden, QW = c.heads * c.head_dim, KW = c.kv_heads * c.head_dim;
+  DENSE_HIP(hipSetDevice(D.device), "hipSetDevice");
+  StepRows R{};
+  size_t bytes = 0;
+  auto place = [&](auto** p, size_t n) {
+    *p = reinterpret_cast<std::remove_reference_t<decltype(*p)>>(reinterpret_cast<uintptr_t>(D.work) + bytes);
+    bytes += (n * sizeof(**p) + 255) / 256 * 256;
+  };
+  for (int pass = 0; pass < 2; ++pass) {  // sizes, then addresses
+    bytes = 0;
+    place(&R.hidden, m * H);
+    place(&R.after, m * H);
+    place(&R.next, m * H);
+    place(&R.x, m * std::max(H, QW));
+    place(&R.q, m * QW);
+    place(&R.k, m * KW);
+    place(&R.v, m * KW);
+    place(&R.proj, m * H);
+    place(&R.out, out_bytes(c));
+    if (int st = grow(&D.work, &D.work_cap, bytes, false)) return st;
+  }
+  if (int st = grow(&D.host_in, &D.in_cap, m * H * 2, true)) return st;
+  if (int st = grow(&D.host_out, &D.out_cap, out_bytes(c), true)) return st;
+  if (int st = grow_rope(M, M->position + m, stream)) return st;
+  for (KvCache& kv : M->caches)
+    if (int st = grow_ring(M, kv, M->position, m, stream)) return st;
+  for (size_t r = 0; r < m; ++r)
+    std::memcpy(D.host_in + r * H * 2, M->embedding + (size_t)tokens[r] * H, H * 2);
+  const int st = enqueue_step(M, m, R, stream);
   if (st != GOSSMX_OK) {
     (void)hipStreamSynchronize(stream);  // the staging buffers' copies end before the next step reuses them
     return st;
   }
-  std::memcpy(hidden, h_rows + n, n * 2);
+  DENSE_HIP(hipStreamSynchronize(stream), "model step");
+  const gossmx::ModelMark* marks = reinterpret_cast<const gossmx::ModelMark*>(D.host_out);
+  uint64_t ticks = 0;
+  for (size_t li = 0; li < c.layers; ++li) {
+    if (marks[li].flags) return gossmx::error_flags_result(M->ctx, marks[li].flags);
+    ticks += marks[li].end - marks[li].begin;
+  }
+  *moe = (double)ticks / D.clock_hz;
   return GOSSMX_OK;
-}
-
-int gpu_o_residual_moe(gossmx_model* M, const gossmx_dense_layer& L, const DenseDevice::Layer& DL,
-                       const uint16_t* attn, size_t m, uint16_t* hidden, double* moe) {
-  return gossmx::run_time_result(M->ctx, gpu_o_residual_moe_impl(M, L, DL, attn, m, hidden, moe));
 }
 
 // One layer-major step over m rows at positions model->position + r
 // (prepare_step with every row in one sequence). Writes the last row's logits.
-// The caches change only when the step succeeds.
+// The caches change only when the step succeeds. A run-time failure on the GPU
+// (HIP error, out of memory) opens the circuit breaker, as a failed projection
+// call does.
 int run_step(gossmx_model* M, const uint32_t* tokens, size_t m, float* logits) {
   const gossmx_model_config& c = M->cfg;
-  const size_t H = c.hidden, QW = c.heads * c.head_dim, KW = c.kv_heads * c.head_dim;
   for (size_t r = 0; r < m; ++r)
     if (tokens[r] >= c.vocab) return err(GOSSMX_ERR_INVALID_ARGUMENT, "token id is not below vocab");
   if (M->position + m > c.context_cap)
     return err(GOSSMX_ERR_INVALID_DIMENSIONS, "the step would pass the sequence's context cap");
   const auto t_step = std::chrono::steady_clock::now();
   double moe = 0.0;
-  const size_t base = M->position;
-  std::vector<uint16_t> hidden(m * H), normalized(m * H), attn(m * QW);
-  std::vector<float> q(m * QW), k(m * KW), v(m * KW), attn_f(m * QW), scores;
-  std::vector<uint16_t> staged_k(c.layers * m * KW), staged_v(c.layers * m * KW);
-  for (size_t r = 0; r < m; ++r) std::memcpy(&hidden[r * H], M->embedding + (size_t)tokens[r] * H, H * 2);
-  Pool& pool = *M->pool;
-  for (size_t li = 0; li < c.layers; ++li) {
-    const gossmx_dense_layer& L = M->layers[li];
-    const DenseDevice::Layer& DL = M->dev.layers[li];
-    const KvCache& cache = M->caches[li];
-    pool.run(m, [&](size_t r) { norm_boundary(&hidden[r * H], L.input_norm, H, c.rms_norm_eps, &normalized[r * H]); });
-    const Projection qkv[3] = {{DL.q, DL.qb, QW, q.data()}, {DL.k, DL.kb, KW, k.data()}, {DL.v, DL.vb, KW, v.data()}};
-    if (int st = gpu_project(M, normalized.data(), m, H, qkv, 3)) return st;
-    uint16_t* sk = &staged_k[li * m * KW];
-    uint16_t* sv = &staged_v[li * m * KW];
-    // Rows are independent once staged: row r attends to the committed rows and
-    // the staged rows 0..r of this step.
-    pool.run(m, [&](size_t r) {
-      float* qr = &q[r * QW];
-      float* kr = &k[r * KW];
-      for (size_t i = 0; i < QW; ++i) qr[i] = bf16_round(qr[i]);
-      for (size_t i = 0; i < KW; ++i) kr[i] = bf16_round(kr[i]);
-      rope_apply(M->rope, qr, c.heads, base + r);
-      rope_apply(M->rope, kr, c.kv_heads, base + r);
-      for (size_t i = 0; i < KW; ++i) {
-        sk[r * KW + i] = bf16_bits(kr[i]);
-        sv[r * KW + i] = bf16_bits(v[r * KW + i]);
-      }
-    });
-    // Tasks of (row, block of heads): a one-row step still spreads over the
-    // pool.
-    const size_t head_blocks = std::min<size_t>(c.heads, m >= 16 ? 1 : (32 + m - 1) / m);
-    const size_t per_block = (c.heads + head_blocks - 1) / head_blocks;
-    pool.run(m * head_blocks, [&](size_t task) {
-      thread_local std::vector<float> sc;
-      const size_t r = task / head_blocks, hb = task % head_blocks;
-      const size_t h_begin = hb * per_block, h_end = std::min(c.heads, h_begin + per_block);
-      if (h_begin >= h_end) return;
-      // Positions below `base` are committed (slot p % capacity of the ring),
-      // the others are this step's staged rows.
-      const size_t combined = cache.len + r + 1;
-      const size_t visible = std::min(combined, cache.capacity);
-      const size_t first = base + r + 1 - visible, cap = cache.capacity;
-      const uint16_t* ck = cache.k.data();
-      const uint16_t* cv = cache.v.data();
-      const uint16_t* rk = sk;
-      const uint16_t* rv = sv;
-      auto key = [=](size_t t) -> const uint16_t* {
-        const size_t p = first + t;
-        return p < base ? ck + (p % cap) * KW : rk + (p - base) * KW;
-      };
-      auto value = [=](size_t t) -> const uint16_t* {
-        const size_t p = first + t;
-        return p < base ? cv + (p % cap) * KW : rv + (p - base) * KW;
-      };
-      float* ctx = &attn_f[r * QW];
-      attention(&q[r * QW], visible, key, value, L.sinks, c.heads, c.kv_heads, c.head_dim, ctx, sc, h_begin, h_end);
-      for (size_t i = h_begin * c.head_dim; i < h_end * c.head_dim; ++i) attn[r * QW + i] = bf16_bits(ctx[i]);
-    });
-    // O projection, residual add and the MoE half (norm_boundary(after,
-    // post_attention_norm), moe_batch, add_residual) -> the next layer's rows.
-    // The MoE block's profile records carry the layer and the phase.
-    (void)gossmx_profile_tag(M->ctx, (int)li, base == 0 || m > 1 ? GOSSMX_PHASE_PREFILL : GOSSMX_PHASE_DECODE);
-    const int st = gpu_o_residual_moe(M, L, DL, attn.data(), m, hidden.data(), &moe);
-    if (st != GOSSMX_OK) return st;
-  }
-  // Final norm and lm_head for the last row (the only row whose logits are required).
-  std::vector<uint16_t> fin(H);
-  norm_boundary(&hidden[(m - 1) * H], M->final_norm, H, c.rms_norm_eps, fin.data());
-  const Projection head = {M->dev.lm_head, nullptr, c.vocab, logits};
-  if (int st = gpu_project(M, fin.data(), 1, H, &head, 1)) return st;
-  bool finite = true;
+  if (int st = gossmx::run_time_result(M->ctx, gpu_step(M, tokens, m, &moe))) return st;
+  // The logits are bf16 values; an exponent of all ones is an infinity or a NaN.
+  const uint16_t* bits =
+      reinterpret_cast<const uint16_t*>(M->dev.host_out + c.layers * sizeof(gossmx::ModelMark));
+  uint32_t not_finite = 0;
   for (size_t i = 0; i < c.vocab; ++i) {
-    logits[i] = bf16_round(logits[i]);
-    finite = finite && std::isfinite(logits[i]);
+    not_finite |= (bits[i] & 0x7f80u) == 0x7f80u;
+    logits[i] = bf16_f32(bits[i]);
   }
-  if (!finite) return err(GOSSMX_ERR_NON_FINITE_LOGITS, "CPU model produced non-finite logits");
-  // Commit the staged rows.
-  for (size_t li = 0; li < c.layers; ++li)
-    for (size_t r = 0; r < m; ++r)
-      M->caches[li].append(base + r, &staged_k[(li * m + r) * KW], &staged_v[(li * m + r) * KW]);
-  M->position = base + m;
+  if (not_finite) return err(GOSSMX_ERR_NON_FINITE_LOGITS, "CPU model produced non-finite logits");
+  // Commit the step's rows.
+  for (KvCache& kv : M->caches)
+    for (size_t r = 0; r < m; ++r) kv.append(M->position + r);
+  M->position += m;
   M->moe_seconds += moe;
-  M->dense_seconds += seconds_since(t_step) - moe;
+  M->dense_seconds += std::max(0.0, seconds_since(t_step) - moe);
   return GOSSMX_OK;
 }
 
+// Empty caches; the rings stay allocated.
 void reset_caches(gossmx_model* M) {
-  const size_t KW = M->cfg.kv_heads * M->cfg.head_dim;
-  M->caches.assign(M->cfg.layers, KvCache{});
+  M->caches.resize(M->cfg.layers);
   for (size_t li = 0; li < M->cfg.layers; ++li) {
     KvCache& kv = M->caches[li];
     kv.capacity = M->layers[li].sliding ? M->cfg.sliding_window : M->cfg.context_cap;
-    kv.width = KW;
+    kv.len = kv.start = 0;
   }
   M->position = 0;
 }
@@ -626,19 +568,17 @@ int gossmx_model_create(gossmx_ctx* ctx, const gossmx_model_config* config, cons
   M->ctx = ctx;
   M->cfg = *config;
   M->embedding = embedding;
-  M->final_norm = final_norm;
-  M->lm_head = lm_head;
   M->layers.assign(layers, layers + config->layers);
   M->rope = make_rope(*config);
-  size_t threads = config->threads;
-  if (!threads) threads = std::max(1u, std::thread::hardware_concurrency());
-  M->pool.reset(new Pool(std::min<size_t>(threads, 64)));
   reset_caches(M);
-  // The projection weights and lm_head go to the context's GPU.
+  // The dense tensors but the embedding go to the context's GPU.
   const size_t H = config->hidden, QW = config->heads * config->head_dim, KW = config->kv_heads * config->head_dim;
   DenseDevice& D = M->dev;
   D.device = gossmx::context_device(ctx);
   int st = hipSetDevice(D.device) == hipSuccess ? GOSSMX_OK : err(GOSSMX_ERR_DEVICE, "hipSetDevice failed");
+  int khz = 0;
+  if (st == GOSSMX_OK && hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, D.device) == hipSuccess && khz > 0)
+    D.clock_hz = 1e3 * khz;
   D.layers.resize(config->layers);
   for (size_t li = 0; li < config->layers && st == GOSSMX_OK; ++li) {
     const gossmx_dense_layer& L = layers[li];
@@ -651,8 +591,11 @@ int gossmx_model_create(gossmx_ctx* ctx, const gossmx_model_config* config, cons
     if (!st) st = upload(D, L.k_bias, KW, &DL.kb);
     if (!st) st = upload(D, L.v_bias, KW, &DL.vb);
     if (!st) st = upload(D, L.o_bias, H, &DL.ob);
+    if (!st) st = upload(D, L.input_norm, H, &DL.input_norm);
     if (!st) st = upload(D, L.post_attention_norm, H, &DL.post_norm);
+    if (!st) st = upload(D, L.sinks, config->heads, &DL.sinks);
   }
+  if (!st) st = upload(D, final_norm, H, &D.final_norm);
   if (!st) st = upload(D, lm_head, config->vocab * H, &D.lm_head);
   if (st) {
     delete M;
@@ -712,10 +655,23 @@ int gossmx_model_times(const gossmx_model* model, double* dense_seconds, double*
 
 int gossmx_greedy_token(const float* logits, size_t n, uint32_t* token) {
   if (!logits || !token) return err(GOSSMX_ERR_INVALID_ARGUMENT, "null argument");
-  size_t best = n;
-  for (size_t i = 0; i < n; ++i)
-    if (std::isfinite(logits[i]) && (best == n || logits[i] > logits[best])) best = i;
-  if (best == n) return err(GOSSMX_ERR_NON_FINITE_LOGITS, "model returned no finite logits");
+  // A pass over integers that the compiler vectorizes: the bits of a finite
+  // float as an int of the same order (-0.0 as +0.0), the lowest int for the
+  // others. Then the first index that holds the largest.
+  constexpr int32_t kNone = INT32_MIN;
+  auto key = [](float f) -> int32_t {
+    const int32_t b = (int32_t)f2u(f), magnitude = b & 0x7fffffff;
+    const int32_t ordered = b < 0 ? -magnitude : magnitude;
+    return magnitude < 0x7f800000 ? ordered : kNone;
+  };
+  int32_t largest = kNone;
+  for (size_t i = 0; i < n; ++i) {
+    const int32_t v = key(logits[i]);
+    largest = v > largest ? v : largest;
+  }
+  if (largest == kNone) return err(GOSSMX_ERR_NON_FINITE_LOGITS, "model returned no finite logits");
+  size_t best = 0;
+  while (key(logits[best]) != largest) ++best;
   *token = (uint32_t)best;
   return GOSSMX_OK;
 }
@@ -737,10 +693,7 @@ int gossmx_attention(const float* query, const uint16_t* keys, const uint16_t* v
   if (!heads || !kv_heads || heads % kv_heads || !head_dim || !window)
     return err(GOSSMX_ERR_INVALID_DIMENSIONS, "invalid CPU attention dimensions");
   const size_t visible = std::min(tokens, window), first = tokens - visible, KW = kv_heads * head_dim;
-  std::vector<float> scores;
-  attention(query, visible, [&](size_t t) { return keys + (first + t) * KW; },
-            [&](size_t t) { return values + (first + t) * KW; }, sinks, heads, kv_heads, head_dim, out, scores, 0,
-            heads);
+  attention(query, visible, keys + first * KW, values + first * KW, sinks, heads, kv_heads, head_dim, out);
   return GOSSMX_OK;
 }
 

@@ -276,9 +276,41 @@ hipError_t launch_dense_proj(const DenseSet& set, int count, const float* x, int
 // One token through up to three projections with the whole K range of a
 // work-group staged at once (cols a multiple of 8, at most 4096).
 hipError_t launch_dense_gemv(const DenseSet& set, int count, const float* x, int cols, hipStream_t stream);
-// after[i] = bf16(hidden[i] + bf16(proj[i])) for i < n (bf16 bits).
-hipError_t launch_residual_add(const uint16_t* hidden, const float* proj, uint16_t* after, size_t n,
+// lm_head of one row: logits[o] = bf16(dot(w[o], x)) for o < rows.
+hipError_t launch_lm_head(const uint16_t* w, const float* x, uint16_t* logits, int rows, int cols,
+                          hipStream_t stream);
+// A layer's MoE call as the device saw it: the clock (wall_clock64) before and
+// after it, and the context's error flags after it.
+struct ModelMark {
+  uint64_t begin, end;
+  int flags, pad;
+};
+// after[i] = bf16(hidden[i] + bf16(proj[i])) for i < n (bf16 bits); *stamp =
+// the device clock.
+hipError_t launch_residual_add(const uint16_t* hidden, const float* proj, uint16_t* after, size_t n, uint64_t* stamp,
                                hipStream_t stream);
+// norm_boundary of the m rows of x (n bf16 values each) by w, as f32; with
+// `mark`, mark->end and mark->flags (= *err) are set first.
+hipError_t launch_dense_norm(const uint16_t* x, const float* w, int m, int n, float eps, float* out, ModelMark* mark,
+                             const int* err, hipStream_t stream);
+// One layer's attention over m rows at positions base + r. Position p's key
+// and value rows (kv_heads x head_dim bf16) live in slot p % slots of k and v;
+// `len` positions before base are committed, and row r sees the last
+// min(len + r + 1, capacity) positions up to its own, which slots >=
+// min(base, capacity - 1) + m keeps apart.
+struct AttnArgs {
+  float* q;            // [m][heads][head_dim] projections; rotated in place
+  const float* k_new;  // [m][kv_heads][head_dim] projections of the m rows
+  const float* v_new;
+  const float* rope;  // [position][head_dim]: bf16 cosines, then sines, of each frequency
+  uint16_t *k, *v;    // the ring; the m rows are stored here
+  const float* sinks;  // [heads]
+  float* out;          // [m][heads][head_dim], bf16 values
+  size_t base, len, capacity, slots;
+  int m, heads, kv_heads, head_dim;
+  float scale;
+};
+hipError_t launch_attention(const AttnArgs& a, hipStream_t stream);
 
 }  // namespace gossmx
 
@@ -295,6 +327,10 @@ int set_error(int status, const char* message);
 const gossmx_moe_config* layer_config(const gossmx_layer* layer);
 int context_device(const gossmx_ctx* ctx);
 hipStream_t context_stream(const gossmx_ctx* ctx);
+// The context's device error flags, and the status of a value read from them
+// (cleared when not zero).
+const int* context_error_flags(const gossmx_ctx* ctx);
+int error_flags_result(gossmx_ctx* ctx, int flags);
 // A GPU round trip's status: GOSSMX_ERR_DEVICE or GOSSMX_ERR_OUT_OF_MEMORY
 // drains the context's stream and opens the process-wide circuit breaker.
 int run_time_result(gossmx_ctx* ctx, int status);

@@ -4299,7 +4299,8 @@ __device__ __forceinline__ void dense_load(DenseChunk<TOK>& c, const uint16_t* w
 
 // Work-group columns [wg_begin[p], wg_begin[p + 1]) serve projection p of
 // `set` (up to three projections of the same input in one launch).
-template <int TOK>
+// With LOGITS the outputs are stored as bf16 (lm_head's round trip).
+template <int TOK, bool LOGITS = false>
 __global__ __launch_bounds__(256) void dense_proj_kernel(DenseSet set, const float* __restrict__ x, int cols, int m) {
   static_assert(kDenseRows * 16 == 256 && kDenseKc % 16 == 0 && TOK <= 16, "thread map");
   __shared__ __align__(16) uint16_t s_w[kDenseRows * kDenseWStride];
@@ -4356,7 +4357,10 @@ __global__ __launch_bounds__(256) void dense_proj_kernel(DenseSet set, const flo
 #pragma unroll
       for (int q = 0; q < 16; ++q) s = s + v[q];
       if (bias != nullptr) s = s + bias[o];
-      out[(size_t)r * rows + o] = s;
+      if (LOGITS)
+        reinterpret_cast<uint16_t*>(out)[(size_t)r * rows + o] = bf16_bits(s);
+      else
+        out[(size_t)r * rows + o] = s;
     }
   }
 }
@@ -4443,18 +4447,326 @@ hipError_t launch_dense_gemv(const DenseSet& set, int count, const float* x, int
 
 // The attention half's residual add (add_residual, cpu_runner.rs:3732-3738,
 // after the O projection's bf16 round trip): after = bf16(hidden + bf16(proj)).
+// Its first thread notes the device clock: the layer's MoE call follows.
 __global__ __launch_bounds__(256) void residual_add_kernel(const uint16_t* __restrict__ hidden,
                                                            const float* __restrict__ proj, uint16_t* __restrict__ after,
-                                                           size_t n) {
+                                                           size_t n, uint64_t* stamp) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) after[i] = bf16_bits(bf16_to_f32(hidden[i]) + bf16r(proj[i]));
+  if (i == 0) *stamp = wall_clock64();
 }
 
-hipError_t launch_residual_add(const uint16_t* hidden, const float* proj, uint16_t* after, size_t n,
+hipError_t launch_residual_add(const uint16_t* hidden, const float* proj, uint16_t* after, size_t n, uint64_t* stamp,
                                hipStream_t stream) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(residual_add_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, hidden, proj, after,
-                     n);
+                     n, stamp);
+  return hipGetLastError();
+}
+
+// norm_boundary (cpu_runner.rs:2680-2687) of one row per work-group, as the
+// f32 values of its bf16 results: lane l < 16 sums x_i * x_i over i = l (mod
+// 16) in order, the lanes are added 0..15, y = bf16((x * inverse) * w). The
+// row moves through LDS in pieces of kDenseNormPiece values, so any width is
+// taken. The 16 chains of n / 16 steps bound it; the rows are few (one in a
+// decode step). With `mark` the first work-group also closes the previous
+// layer's MoE call: the device clock, and the error flags as that call left
+// them.
+constexpr int kDenseNormPiece = 4096;  // a multiple of 16
+
+__global__ __launch_bounds__(256) void dense_norm_kernel(const uint16_t* __restrict__ x, const float* __restrict__ w,
+                                                         int n, float eps, float* __restrict__ out, ModelMark* mark,
+                                                         const int* err) {
+  __shared__ __align__(16) uint16_t s_row[kDenseNormPiece];
+  __shared__ float s_lane[16];
+  const int tid = threadIdx.x;
+  const uint16_t* xr = x + (size_t)blockIdx.x * n;
+  if (mark != nullptr && blockIdx.x == 0 && tid == 0) {
+    mark->end = wall_clock64();
+    mark->flags = *err;
+  }
+  float acc = 0.0f;
+  for (int c0 = 0; c0 < n; c0 += kDenseNormPiece) {  // uniform
+    const int len = min(kDenseNormPiece, n - c0);
+    __syncthreads();
+    if ((n & 7) == 0) {
+      for (int v = tid; v < len / 8; v += 256)
+        reinterpret_cast<u32x4*>(s_row)[v] = reinterpret_cast<const u32x4*>(xr + c0)[v];
+    } else {
+      for (int i = tid; i < len; i += 256) s_row[i] = xr[c0 + i];
+    }
+    __syncthreads();
+    if (tid < 16) {
+#pragma unroll 16
+      for (int i = tid; i < len; i += 16) {
+        const float v = bf16_to_f32(s_row[i]);
+        acc = acc + v * v;
+      }
+    }
+  }
+  if (tid < 16) s_lane[tid] = acc;
+  __syncthreads();
+  float ss = 0.0f;
+#pragma unroll
+  for (int l = 0; l < 16; ++l) ss = ss + s_lane[l];
+  const float inv = 1.0f / sqrtf(ss / (float)n + eps);
+  float* o = out + (size_t)blockIdx.x * n;
+  for (int i = tid; i < n; i += 256) {
+    // A row of one piece is still in LDS.
+    const float v = bf16_to_f32(n <= kDenseNormPiece ? s_row[i] : xr[i]);
+    o[i] = bf16r(v * inv * w[i]);
+  }
+}
+
+hipError_t launch_dense_norm(const uint16_t* x, const float* w, int m, int n, float eps, float* out, ModelMark* mark,
+                             const int* err, hipStream_t stream) {
+  if (m <= 0 || n <= 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(dense_norm_kernel, dim3((unsigned)m), dim3(256), 0, stream, x, w, n, eps, out, mark, err);
+  return hipGetLastError();
+}
+
+// The bf16 round trips of a step's Q, K and V rows, YaRN RoPE of Q and K with
+// its bf16 boundaries (YarnRope::apply, cpu_runner.rs:3966-4013), and the
+// store of the key and value rows into the layer's ring: position p in slot
+// p % slots. Items of row r: heads x half rotations of Q (in place, f32), then
+// kv_heads x half rotations of K, then the V pairs. The cosines and sines
+// (bf16 values) come from the host's table, row per position.
+__global__ __launch_bounds__(256) void qkv_finish_kernel(AttnArgs a) {
+  const int half = a.head_dim / 2, q_items = a.heads * half, k_items = a.kv_heads * half;
+  const int per_row = q_items + 2 * k_items;
+  const size_t total = (size_t)a.m * per_row, step = (size_t)gridDim.x * 256;
+  const size_t KW = (size_t)a.kv_heads * a.head_dim;
+  for (size_t it = (size_t)blockIdx.x * 256 + threadIdx.x; it < total; it += step) {
+    const size_t r = it / per_row;
+    int i = (int)(it - r * per_row);
+    const size_t p = a.base + r, slot = (p % a.slots) * KW;
+    if (i < q_items + k_items) {
+      const bool is_q = i < q_items;
+      if (!is_q) i -= q_items;
+      const int h = i / half, d = i - h * half;
+      const float* row = is_q ? a.q + r * a.heads * a.head_dim : a.k_new + r * KW;
+      const float* t = a.rope + p * a.head_dim;
+      const float cosine = t[d], sine = t[half + d];
+      const float left = bf16r(row[h * a.head_dim + d]), right = bf16r(row[h * a.head_dim + half + d]);
+      const float x = bf16r(left * cosine) - bf16r(right * sine), y = bf16r(right * cosine) + bf16r(left * sine);
+      if (is_q) {
+        float* o = a.q + r * a.heads * a.head_dim + h * a.head_dim;
+        o[d] = bf16r(x);
+        o[half + d] = bf16r(y);
+      } else {
+        uint16_t* o = a.k + slot + h * a.head_dim;
+        o[d] = bf16_bits(x);
+        o[half + d] = bf16_bits(y);
+      }
+    } else {
+      const int e = 2 * (i - q_items - k_items);
+      const float* v = a.v_new + r * KW + e;
+      *reinterpret_cast<uint32_t*>(a.v + slot + e) = (uint32_t)bf16_bits(v[0]) | ((uint32_t)bf16_bits(v[1]) << 16);
+    }
+  }
+}
+
+// Attention with learned sinks (attention_one_staged, cpu_runner.rs:3840-3924):
+// a work-group computes HEADS query heads of one kv head for one row, over the
+// row's visible window of the ring. Every float chain is the reference's: a
+// score is one thread's dot over d in order, rounded to bf16, scaled and
+// rounded again; one thread per head adds the exponentials in token order; one
+// thread per (head, pair of values) adds p * v in token order, each product
+// and sum rounded by itself. What bounds it is the token-order chains, so the
+// heads of a kv head share a work-group (its keys and values are read once for
+// 8 heads) where that still gives every CU a work-group, and take one each
+// where it does not: 64 heads of 64 values, 8 kv heads, 63 rows 21.6 us shared
+// and 37 us apart, one row 21.6 us shared and 12.5 us apart. Scores live in LDS, kAttnScores at a time: a window
+// that fits is scored once, a longer one once per pass (maximum, sum, values),
+// so any window is taken without a scratch buffer.
+constexpr int kAttnScores = 8192;  // scores in LDS per work-group (32 KB): 8,192 tokens of 1 head, 1,024 of 8
+constexpr int kAttnQ = 128;        // query values per head in LDS
+constexpr int kAttnAhead = 32;     // value rows in flight per thread
+constexpr size_t kAttnSharedMin = 256;  // work-groups (one per CU) from which 8 heads share one
+
+template <int HEADS>
+__global__ __launch_bounds__(256) void attention_kernel(AttnArgs a) {
+  constexpr int kTokens = kAttnScores / HEADS, kStride = kTokens + 4;
+  __shared__ __align__(16) float s_q[HEADS * kAttnQ];
+  __shared__ __align__(16) float s_s[HEADS * kStride];
+  __shared__ uint64_t s_tab[32];
+  __shared__ float s_wave[4 * HEADS], s_max[HEADS], s_den[HEADS];
+  const int tid = threadIdx.x, hd = a.head_dim, half = hd / 2;
+  const int groups = a.heads / a.kv_heads, blocks = (groups + HEADS - 1) / HEADS;
+  const int hb = (int)(blockIdx.x % blocks), kvh = (int)(blockIdx.x / blocks % a.kv_heads);
+  const size_t r = blockIdx.x / blocks / a.kv_heads, KW = (size_t)a.kv_heads * hd;
+  const int h0 = kvh * groups + hb * HEADS, nh = min(HEADS, groups - hb * HEADS);
+  const int visible = (int)min(a.len + r + 1, a.capacity);
+  const size_t first = (a.base + r + 1 - visible) % a.slots;
+  const float* q = a.q + (r * a.heads + h0) * hd;
+  float* out = a.out + (r * a.heads + h0) * hd;
+  const uint16_t* kp = a.k + (size_t)kvh * hd;
+  const uint16_t* vp = a.v + (size_t)kvh * hd;
+  auto slot = [&](int t) -> size_t {
+    const size_t s = first + t;
+    return (s < a.slots ? s : s - a.slots) * KW;
+  };
+  if (tid < 32) s_tab[tid] = kExp2Tab[tid];
+  bool staged = false;
+  float mx[HEADS];
+#pragma unroll
+  for (int h = 0; h < HEADS; ++h) mx[h] = a.sinks[h0 + min(h, nh - 1)];
+  // Scores of the tokens [t0, t0 + n) into s_s; ends with a barrier.
+  auto score = [&](int t0, int n) {
+    for (int j0 = 0; j0 < n; j0 += 256) {  // uniform
+      const int j = j0 + tid;
+      const bool live = j < n;
+      const uint16_t* k = kp + slot(t0 + min(j, n - 1));
+      float acc[HEADS];
+#pragma unroll
+      for (int h = 0; h < HEADS; ++h) acc[h] = 0.0f;
+      for (int d0 = 0; d0 < hd; d0 += kAttnQ) {  // uniform
+        const int dn = min(kAttnQ, hd - d0);
+        if (!staged || hd > kAttnQ) {
+          __syncthreads();
+          for (int i = tid; i < HEADS * dn; i += 256) {
+            const int h = i / dn, d = i - h * dn;
+            s_q[h * kAttnQ + d] = q[(size_t)min(h, nh - 1) * hd + d0 + d];
+          }
+          staged = true;
+          __syncthreads();
+        }
+        if (live && (hd & 7) == 0) {
+#pragma unroll 8
+          for (int d = 0; d < dn; d += 8) {
+            const u32x4 kv = *reinterpret_cast<const u32x4*>(k + d0 + d);
+            float kf[8];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              kf[2 * e] = __uint_as_float(kv[e] << 16);
+              kf[2 * e + 1] = __uint_as_float(kv[e] & 0xffff0000u);
+            }
+#pragma unroll
+            for (int h = 0; h < HEADS; ++h)
+#pragma unroll
+              for (int e = 0; e < 8; ++e) acc[h] = acc[h] + s_q[h * kAttnQ + d + e] * kf[e];
+          }
+        } else if (live) {
+          for (int d = 0; d < dn; ++d) {
+            const float kf = bf16_to_f32(k[d0 + d]);
+#pragma unroll
+            for (int h = 0; h < HEADS; ++h) acc[h] = acc[h] + s_q[h * kAttnQ + d] * kf;
+          }
+        }
+      }
+      if (live) {
+#pragma unroll
+        for (int h = 0; h < HEADS; ++h) s_s[h * kStride + j] = bf16r(bf16r(acc[h]) * a.scale);
+      }
+    }
+    __syncthreads();
+  };
+  const bool single = visible <= kTokens;
+  for (int t0 = 0; t0 < visible; t0 += kTokens) {  // uniform
+    const int n = min(kTokens, visible - t0);
+    score(t0, n);
+    for (int j = tid; j < n; j += 256) {
+#pragma unroll
+      for (int h = 0; h < HEADS; ++h) mx[h] = fmaxf(mx[h], s_s[h * kStride + j]);
+    }
+    if (!single) __syncthreads();  // the next chunk overwrites the scores
+  }
+#pragma unroll
+  for (int h = 0; h < HEADS; ++h) {
+#pragma unroll
+    for (int x = 32; x >= 1; x >>= 1) mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], x));
+    if ((tid & 63) == 0) s_wave[(tid >> 6) * HEADS + h] = mx[h];
+  }
+  __syncthreads();
+  if (tid < HEADS)
+    s_max[tid] = fmaxf(fmaxf(s_wave[tid], s_wave[HEADS + tid]), fmaxf(s_wave[2 * HEADS + tid], s_wave[3 * HEADS + tid]));
+  __syncthreads();
+  // s_s[h][j] = expf(score - maximum), for j < n; ends with a barrier.
+  auto exponentials = [&](int n) {
+    for (int j = tid; j < n; j += 256) {
+#pragma unroll
+      for (int h = 0; h < HEADS; ++h) s_s[h * kStride + j] = expf_glibc(s_s[h * kStride + j] - s_max[h], s_tab);
+    }
+    __syncthreads();
+  };
+  float sum = 0.0f;
+  for (int t0 = 0; t0 < visible; t0 += kTokens) {  // uniform
+    const int n = min(kTokens, visible - t0);
+    if (!single) score(t0, n);
+    exponentials(n);
+    if (tid < HEADS) {
+#pragma unroll 16
+      for (int j = 0; j < n; ++j) sum = sum + s_s[tid * kStride + j];
+    }
+    if (!single) __syncthreads();
+  }
+  if (tid < HEADS) s_den[tid] = expf_glibc(a.sinks[h0 + min(tid, nh - 1)] - s_max[tid], s_tab) + sum;
+  __syncthreads();
+  for (int t0 = 0; t0 < visible; t0 += kTokens) {  // uniform
+    const int n = min(kTokens, visible - t0);
+    if (!single) {
+      score(t0, n);
+      exponentials(n);
+    }
+    for (int j = tid; j < n; j += 256) {
+#pragma unroll
+      for (int h = 0; h < HEADS; ++h) s_s[h * kStride + j] = bf16r(s_s[h * kStride + j] / s_den[h]);
+    }
+    __syncthreads();
+    const bool last = t0 + n == visible;
+    for (int i = tid; i < nh * half; i += 256) {
+      const int h = i / half, d = 2 * (i - h * half);
+      float* o = out + (size_t)h * hd + d;
+      const float* p = &s_s[h * kStride];
+      float x = 0.0f, y = 0.0f;
+      if (t0 != 0) {
+        x = o[0];
+        y = o[1];
+      }
+      int j = 0;
+      for (; j + kAttnAhead <= n; j += kAttnAhead) {
+        uint32_t v[kAttnAhead];
+#pragma unroll
+        for (int u = 0; u < kAttnAhead; ++u) v[u] = *reinterpret_cast<const uint32_t*>(vp + slot(t0 + j + u) + d);
+#pragma unroll
+        for (int u = 0; u < kAttnAhead; ++u) {
+          x = x + p[j + u] * __uint_as_float(v[u] << 16);
+          y = y + p[j + u] * __uint_as_float(v[u] & 0xffff0000u);
+        }
+      }
+      if (j < n) {
+        uint32_t v[kAttnAhead];
+#pragma unroll
+        for (int u = 0; u < kAttnAhead; ++u)
+          v[u] = *reinterpret_cast<const uint32_t*>(vp + slot(t0 + min(j + u, n - 1)) + d);
+#pragma unroll
+        for (int u = 0; u < kAttnAhead; ++u) {
+          if (j + u < n) {
+            x = x + p[j + u] * __uint_as_float(v[u] << 16);
+            y = y + p[j + u] * __uint_as_float(v[u] & 0xffff0000u);
+          }
+        }
+      }
+      o[0] = last ? bf16r(x) : x;
+      o[1] = last ? bf16r(y) : y;
+    }
+    if (!last) __syncthreads();
+  }
+}
+
+hipError_t launch_attention(const AttnArgs& a, hipStream_t stream) {
+  if (a.m <= 0 || a.heads <= 0 || a.kv_heads <= 0 || a.heads % a.kv_heads || a.head_dim <= 0 || a.head_dim % 2 ||
+      a.capacity == 0 || a.len > a.base || a.slots < std::min(a.base, a.capacity - 1) + (size_t)a.m)
+    return hipErrorInvalidValue;
+  const size_t items = (size_t)a.m * (a.heads + 2 * a.kv_heads) * (a.head_dim / 2);
+  hipLaunchKernelGGL(qkv_finish_kernel, dim3((unsigned)std::min<size_t>((items + 255) / 256, 8192)), dim3(256), 0,
+                     stream, a);
+  const int groups = a.heads / a.kv_heads;
+  const size_t shared = (size_t)a.m * a.kv_heads * ((groups + 7) / 8);
+  if (groups > 1 && shared >= kAttnSharedMin)
+    hipLaunchKernelGGL(attention_kernel<8>, dim3((unsigned)shared), dim3(256), 0, stream, a);
+  else
+    hipLaunchKernelGGL(attention_kernel<1>, dim3((unsigned)((size_t)a.m * a.heads)), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -4475,6 +4787,19 @@ hipError_t launch_dense_proj(const DenseSet& set, int count, const float* x, int
   else
     hipLaunchKernelGGL(dense_proj_kernel<16>, dim3((unsigned)wg, (unsigned)((m + 15) / 16)), dim3(256), 0, stream, s,
                        x, cols, m);
+  return hipGetLastError();
+}
+
+hipError_t launch_lm_head(const uint16_t* w, const float* x, uint16_t* logits, int rows, int cols,
+                          hipStream_t stream) {
+  if (rows <= 0 || cols <= 0) return hipErrorInvalidValue;
+  DenseSet s{};
+  s.w[0] = w;
+  s.out[0] = reinterpret_cast<float*>(logits);
+  s.rows[0] = rows;
+  const int wg = (rows + kDenseRows - 1) / kDenseRows;
+  for (int i = 1; i < 4; ++i) s.wg_begin[i] = wg;
+  hipLaunchKernelGGL((dense_proj_kernel<1, true>), dim3((unsigned)wg, 1), dim3(256), 0, stream, s, x, cols, 1);
   return hipGetLastError();
 }
 

@@ -519,15 +519,14 @@ int gossmx_selftest_bf16_exhaustive(gossmx_ctx* ctx, uint64_t* mismatches);
 /* ---------------------------------------------------------------------------
  * The dense path around the block (crates/gpt-oss-model-runner/src/
  * cpu_runner.rs): a GPT-OSS model that computes what the reference's CPU runner
- * computes, bit for bit. Attention, RoPE, norms and the KV caches run on host
- * threads. The Q/K/V/O projections and lm_head run on the context's GPU with the
- * reference's 16-lane dot order, over copies of those matrices made in HBM by
- * gossmx_model_create (about 2.4 GB for GPT-OSS-20B, with the post-attention
- * norm weights). The MoE halves run on the GPU through
- * gossmx_moe_forward_residual (device memory, one round trip per layer with the
- * O projection). The embedding, the input and final norm weights, the sinks and
- * the MoE layers stay borrowed and must outlive the model. A model holds one
- * sequence's KV caches. */
+ * computes, bit for bit. A step runs on the context's GPU: norms, the Q/K/V/O
+ * projections and lm_head in the reference's 16-lane dot order, RoPE, attention
+ * over KV caches in HBM, and the MoE halves through gossmx_moe_forward_residual;
+ * the host gathers the embedding rows and reads the logits, one synchronization
+ * per step. gossmx_model_create copies the dense tensors but the embedding to
+ * HBM (about 2.4 GB for GPT-OSS-20B). The embedding, the other tensors and the
+ * MoE layers must outlive the model. A model holds one sequence's KV caches;
+ * they grow with the sequence and stay allocated until it is destroyed. */
 typedef struct gossmx_model gossmx_model;
 
 /* CpuGptOssConfig (cpu_runner.rs:252-291) and the sequence's context cap
@@ -549,7 +548,7 @@ typedef struct gossmx_model_config {
   double rope_beta_fast;              /* 32 by default */
   double rope_beta_slow;              /* 1 by default */
   int rope_truncate;
-  size_t threads;                     /* host threads for the dense path; 0: all hardware threads (at most 64) */
+  size_t threads;                     /* host threads of the reference's dense path; the steps need none */
 } gossmx_model_config;
 
 /* One decoder layer (CpuLayer, load_layer cpu_runner.rs:3526-3671). Vectors are
@@ -593,8 +592,8 @@ int gossmx_model_decode(gossmx_model* model, uint32_t token, float* logits);
 int gossmx_model_position(const gossmx_model* model, size_t* position);
 /* CpuKvCache::len / start_position of a layer's cache (:674-680). */
 int gossmx_model_cache(const gossmx_model* model, size_t layer, size_t* len, size_t* start_position);
-/* Wall time spent so far in the dense path and in the MoE calls (including
- * their host<->device copies). */
+/* Wall time spent so far in the steps, by part: the MoE calls (the device's clock
+ * from a layer's residual add to the next norm) and everything else. */
 int gossmx_model_times(const gossmx_model* model, double* dense_seconds, double* moe_seconds);
 
 /* greedy_token (crates/gpt-oss-bench/src/bin/cpu_parity.rs:750-762): the

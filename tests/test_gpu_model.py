@@ -1,5 +1,4 @@
-"""A GPT-OSS model with its attention on the host and its projections and MoE blocks on the GPU
-(gossmx_model_*) against the oracle's whole-model restatement
+"""A GPT-OSS model on the GPU (gossmx_model_*) against the oracle's whole-model restatement
 (oracle_model_generate): greedy tokens and every logits bit, for a small model
 and for configs[3], the random-init GPT-OSS-20B forward (63-token prefill,
 8 greedy decode steps)."""
@@ -112,6 +111,43 @@ def test_small_model_chunked_prefill(tiny):
     for lo in range(0, PROMPT.size, 5):
         logits = model.append(PROMPT[lo:lo + 5])
     assert_bits(logits, want[0])
+
+
+# Attention's edges: windows past the scores that a work-group holds (1,024
+# tokens where 8 heads share it, 8,192 of one head), a window and a ring that
+# wrap and grow between the steps, heads past a group of 8, and query rows wider
+# than their staging (128 values) with and without 16-byte key loads.
+@pytest.mark.parametrize("heads,kv_heads,head_dim,window,steps", [
+    (16, 2, 16, 300, (1, 299, 800)),
+    (2, 2, 2, 100, (40, 8170)),
+    (9, 1, 130, 64, (130, 1, 130)),
+    (6, 2, 136, 3, (90, 1, 300)),
+])
+def test_attention_edges_match_oracle(ctx, heads, kv_heads, head_dim, window, steps):
+    n = sum(steps)
+    cfg = dict(vocab=64, hidden=32, layers=2, heads=heads, kv_heads=kv_heads, head_dim=head_dim, sliding_window=window,
+               context_cap=n + 3, rms_norm_eps=1e-5, **ROPE_20B)
+    w = synth.model_weights(cfg, synth.numpy_normal(np.random.default_rng(8)))
+    hosts = [O.synthetic_layer(8, i, experts=4, hidden=32, intermediate=32, top_k=2) for i in range(cfg["layers"])]
+    for L, h in zip(w["layers"], hosts):
+        L["moe_host"] = h
+    model, keep = build(ctx, cfg, w, hosts)
+    try:
+        oracle = O.ModelHost(cfg, w["embedding"], w["final_norm"], w["lm_head"], w["layers"])
+        prompt = ((np.arange(n, dtype=np.uint32) * 2654435761) >> 7) % 64
+        st, want_tokens, want_logits = O.model_generate(oracle, prompt, 2, threads=8)
+        assert st == O.OK
+        for turn in range(2):  # the second on the rings that the first one grew
+            model.reset()
+            lo = 0
+            for m in steps:
+                logits = model.append(prompt[lo:lo + m])
+                lo += m
+            assert_bits(logits, want_logits[0])
+            for k in range(2):
+                assert_bits(model.decode(want_tokens[k]), want_logits[k + 1])
+    finally:
+        release(model, keep)
 
 
 def test_small_model_failed_step_changes_nothing(tiny):
