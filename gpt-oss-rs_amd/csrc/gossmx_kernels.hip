@@ -3683,37 +3683,51 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* y, const f
 // Reference activation records -> GEMM operand. Q8Block {f32 scale; i8[32]}
 // is 36 bytes, ResidualQ8Block {primary; residual} 72 bytes (lib.rs:732-742).
 
+// The f16 operand: a thread moves 8 codes of one part (two dwords in, 16 bytes
+// out; records and their codes are 4-byte aligned). Q8 records leave zeros in
+// part 1. At 129 rows of 90 blocks the
+// whole matmul call takes 26.8 us; 27.2 us with 32 threads per record, two bytes
+// in and four out each.
 __global__ __launch_bounds__(256) void prep_records_kernel(const uint8_t* rec, int kind, int m, int blocks,
                                                           size_t row_stride, ActBuffers act) {
+  const size_t it = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (it >= (size_t)m * blocks * 8) return;
+  const int hw = (int)(it >> 3), part = (int)(it >> 2) & 1, oct = (int)it & 3;
+  const int r = hw / blocks, b = hw % blocks;
+  const uint8_t* p = rec + ((size_t)r * row_stride + b) * (kind == 2 ? 72 : 36) + part * 36;
+  float scale = 0.0f;
+  uint32_t c[2] = {0u, 0u};
+  if (part == 0 || kind == 2) {
+    scale = *reinterpret_cast<const float*>(p);
+    c[0] = *reinterpret_cast<const uint32_t*>(p + 4 + 8 * oct);
+    c[1] = *reinterpret_cast<const uint32_t*>(p + 8 + 8 * oct);
+  }
+  half8 h;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) h[i] = (_Float16)(float)(int8_t)(c[i >> 2] >> (8 * (i & 3)));
+  const size_t dst = (size_t)hw * 2 + part;
+  *reinterpret_cast<half8*>(act.v + dst * kBlock + 8 * oct) = h;
+  if (oct == 0) act.s[dst] = scale;
+}
+
+// The digit operand (gemm_wide_kernel): 32 lanes per record.
+__global__ __launch_bounds__(256) void prep_digits_kernel(const uint8_t* rec, int kind, int m, int blocks,
+                                                         size_t row_stride, ActBuffers act) {
   const int hw = (blockIdx.x * blockDim.x + threadIdx.x) >> 5;
   const int l32 = threadIdx.x & 31;
   if (hw >= m * blocks) return;
   const int r = hw / blocks, b = hw % blocks;
-  const size_t rsz = kind == 2 ? 72 : 36;
-  const uint8_t* p = rec + ((size_t)r * row_stride + b) * rsz;
-  const float ps = *reinterpret_cast<const float*>(p);
-  const int8_t pq = (int8_t)p[4 + l32];
-  float rs = 0.0f;
-  int8_t rq = 0;
+  const uint8_t* p = rec + ((size_t)r * row_stride + b) * (kind == 2 ? 72 : 36);
+  uint8_t* digits = reinterpret_cast<uint8_t*>(act.v) + (size_t)hw * kDigitRecord;
+  float2 sc;
+  sc.x = *reinterpret_cast<const float*>(p);
+  sc.y = 0.0f;
+  store_digits(digits, (float)(int8_t)p[4 + l32], l32);
   if (kind == 2) {
-    rs = *reinterpret_cast<const float*>(p + 36);
-    rq = (int8_t)p[40 + l32];
+    sc.y = *reinterpret_cast<const float*>(p + 36);
+    store_digits(digits + kDigitRecord / 2, (float)(int8_t)p[40 + l32], l32);
   }
-  if (act.digits) {
-    uint8_t* rec = reinterpret_cast<uint8_t*>(act.v) + ((size_t)r * blocks + b) * kDigitRecord;
-    store_digits(rec, (float)pq, l32);
-    if (kind == 2) store_digits(rec + kDigitRecord / 2, (float)rq, l32);
-  } else {
-    _Float16* dst = act.v + (((size_t)r * blocks + b) * 2) * kBlock;
-    dst[l32] = (_Float16)(float)pq;
-    dst[kBlock + l32] = (_Float16)(float)rq;
-  }
-  if (l32 == 0) {
-    float2 sc;
-    sc.x = ps;
-    sc.y = rs;
-    reinterpret_cast<float2*>(act.s)[(size_t)r * blocks + b] = sc;
-  }
+  if (l32 == 0) reinterpret_cast<float2*>(act.s)[hw] = sc;
 }
 
 // ---------------------------------------------------------------------------
@@ -4145,8 +4159,12 @@ hipError_t launch_combine(const uint16_t* y, const float* weights, int m, int to
 
 hipError_t launch_prep_records(const uint8_t* records, int kind, size_t m, size_t blocks, size_t row_stride,
                                ActBuffers act, int* /*err*/, hipStream_t stream) {
-  hipLaunchKernelGGL(prep_records_kernel, dim3(grid1d(m * blocks * 32, 256)), dim3(256), 0, stream, records, kind,
-                     (int)m, (int)blocks, row_stride, act);
+  if (act.digits)
+    hipLaunchKernelGGL(prep_digits_kernel, dim3(grid1d(m * blocks * 32, 256)), dim3(256), 0, stream, records, kind,
+                       (int)m, (int)blocks, row_stride, act);
+  else
+    hipLaunchKernelGGL(prep_records_kernel, dim3(grid1d(m * blocks * 8, 256)), dim3(256), 0, stream, records, kind,
+                       (int)m, (int)blocks, row_stride, act);
   return hipGetLastError();
 }
 
