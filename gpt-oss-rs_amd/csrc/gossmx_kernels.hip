@@ -4384,60 +4384,70 @@ __global__ __launch_bounds__(256) void dense_proj_kernel(DenseSet set, const flo
 }
 
 // One token, up to three projections of the same input in one launch (Q, K
-// and V): the same dot, with the work-group's 16 weight rows for the whole K
-// range staged in LDS by loads that are all in flight at once, so the
-// work-group waits for one memory round trip instead of one per K chunk.
-// Work-groups [wg_begin[i], wg_begin[i + 1]) serve projection i. cols is a
-// multiple of 8 and at most kDenseGemvMaxCols.
+// and V): the same dot, with the work-group's weight rows for the whole K range
+// staged in LDS by loads that are all in flight at once, so the work-group
+// waits for one memory round trip instead of one per K chunk. Work-groups
+// [wg_begin[i], wg_begin[i + 1]) serve projection i. cols is a multiple of 8 and
+// at most kDenseGemvMaxCols. One wave of 4 rows: the 1,280 work-groups of Q, K
+// and V (5,120 x 2,880) then fit the CUs' LDS at once, five each, and the 720 of
+// O (2,880 x 4,096) three each, where 16-row work-groups ran one per CU in two
+// rounds (320) or left CUs idle (180): 12.6 and 11.8 us a launch, both 15.2 us on
+// average with 16 rows.
 constexpr int kDenseGemvMaxCols = 4096;
-constexpr int kDenseGemvPieces = kDenseRows * kDenseGemvMaxCols / 8 / 256;  // 16-byte weight pieces per thread
+constexpr int kDenseGemvRows = 4;
+constexpr int kDenseGemvPad = 16;  // u16 after an LDS row: rows start at least 8 banks apart for the usual widths
 
-__global__ __launch_bounds__(256) void dense_gemv_kernel(DenseSet set, const float* __restrict__ x, int cols) {
+// PER: 16-byte weight pieces per thread and row, at least cols / 8 / 64.
+template <int PER>
+__global__ __launch_bounds__(kDenseGemvRows * 16) void dense_gemv_kernel(DenseSet set, const float* __restrict__ x,
+                                                                         int cols) {
+  constexpr int R = kDenseGemvRows, T = R * 16;
   extern __shared__ __align__(16) char s_dyn[];
-  __shared__ float s_fold[kDenseRows * 16];
-  const int stride = cols + 8;  // u16 per LDS row
+  __shared__ float s_fold[T];
+  const int stride = cols + kDenseGemvPad;  // u16 per LDS row
   uint16_t* s_w = reinterpret_cast<uint16_t*>(s_dyn);
-  float* s_x = reinterpret_cast<float*>(s_dyn + (size_t)kDenseRows * stride * 2);
+  uint16_t* s_x = s_w + R * stride;  // x as bf16 (its values are)
   const int tid = threadIdx.x, i = tid >> 4, l = tid & 15;
   const int b = (int)blockIdx.x;
   const int pi = b >= set.wg_begin[2] ? 2 : (b >= set.wg_begin[1] ? 1 : 0);
   const uint16_t* w = set.w[pi];
-  const int rows = set.rows[pi], o0 = (b - set.wg_begin[pi]) * kDenseRows;
-  const int per_row = cols >> 3, n_w = kDenseRows * per_row;
-  u32x4 v[kDenseGemvPieces];
+  const int rows = set.rows[pi], o0 = (b - set.wg_begin[pi]) * R, per_row = cols >> 3;
+  // Pieces past the row's end read its last one, rows past the matrix its last row.
+  u32x4 v[R][PER];
 #pragma unroll
-  for (int q = 0; q < kDenseGemvPieces; ++q) {
-    const int p = tid + 256 * q;
-    const int r = p / per_row, k = (p - r * per_row) * 8;
-    v[q] = u32x4{0u, 0u, 0u, 0u};
-    if (p < n_w && o0 + r < rows) v[q] = *reinterpret_cast<const u32x4*>(w + (size_t)(o0 + r) * cols + k);
+  for (int r = 0; r < R; ++r) {
+    const uint16_t* wr = w + (size_t)min(o0 + r, rows - 1) * cols;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) v[r][q] = *reinterpret_cast<const u32x4*>(wr + 8 * min(tid + T * q, per_row - 1));
   }
-  float4 xv[kDenseGemvMaxCols / 4 / 256];
+  u32x4 xv[PER][2];
 #pragma unroll
-  for (int q = 0; q < kDenseGemvMaxCols / 4 / 256; ++q) {
-    const int p = tid + 256 * q;
-    xv[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (p * 4 < cols) xv[q] = *reinterpret_cast<const float4*>(x + p * 4);
-  }
-#pragma unroll
-  for (int q = 0; q < kDenseGemvPieces; ++q) {
-    const int p = tid + 256 * q;
-    const int r = p / per_row, k = (p - r * per_row) * 8;
-    if (p < n_w) *reinterpret_cast<u32x4*>(&s_w[r * stride + k]) = v[q];
+  for (int q = 0; q < PER; ++q) {
+    const float* xp = x + 8 * min(tid + T * q, per_row - 1);
+    xv[q][0] = *reinterpret_cast<const u32x4*>(xp);
+    xv[q][1] = *reinterpret_cast<const u32x4*>(xp + 4);
   }
 #pragma unroll
-  for (int q = 0; q < kDenseGemvMaxCols / 4 / 256; ++q) {
-    const int p = tid + 256 * q;
-    if (p * 4 < cols) *reinterpret_cast<float4*>(&s_x[p * 4]) = xv[q];
+  for (int q = 0; q < PER; ++q) {
+    const int p = tid + T * q;
+    if (p < per_row) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) *reinterpret_cast<u32x4*>(&s_w[r * stride + 8 * p]) = v[r][q];
+      u32x4 h;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        h[e] = (xv[q][e >> 1][2 * (e & 1)] >> 16) | (xv[q][e >> 1][2 * (e & 1) + 1] & 0xffff0000u);
+      *reinterpret_cast<u32x4*>(&s_x[8 * p]) = h;
+    }
   }
   __syncthreads();
   float acc = 0.0f;
   const uint16_t* wr = &s_w[i * stride];
-#pragma unroll 8
-  for (int k = l; k < cols; k += 16) acc = acc + __uint_as_float((uint32_t)wr[k] << 16) * s_x[k];
-  s_fold[i * 16 + l] = acc;
+#pragma unroll 16
+  for (int k = l; k < cols; k += 16) acc = acc + bf16_to_f32(wr[k]) * bf16_to_f32(s_x[k]);
+  s_fold[tid] = acc;
   __syncthreads();
-  if (tid < kDenseRows && o0 + tid < rows) {
+  if (tid < R && o0 + tid < rows) {
     float s = 0.0f;
 #pragma unroll
     for (int q = 0; q < 16; ++q) s = s + s_fold[tid * 16 + q];
@@ -4446,20 +4456,23 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseSet set, const flo
   }
 }
 
-size_t dense_gemv_lds(int cols) { return (size_t)kDenseRows * (cols + 8) * 2 + (size_t)cols * 4; }
-
 hipError_t launch_dense_gemv(const DenseSet& set, int count, const float* x, int cols, hipStream_t stream) {
   if (count <= 0 || count > 3 || cols <= 0 || cols % 8 != 0 || cols > kDenseGemvMaxCols) return hipErrorInvalidValue;
   DenseSet s = set;
   int wg = 0;
   for (int i = 0; i < 3; ++i) {
     s.wg_begin[i] = wg;
-    if (i < count) wg += (s.rows[i] + kDenseRows - 1) / kDenseRows;
+    if (i < count) wg += (s.rows[i] + kDenseGemvRows - 1) / kDenseGemvRows;
   }
   s.wg_begin[3] = wg;
   if (wg == 0) return hipSuccess;
-  hipLaunchKernelGGL(dense_gemv_kernel, dim3((unsigned)wg), dim3(256), (unsigned)dense_gemv_lds(cols), stream, s, x,
-                     cols);
+  const auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)wg), dim3(kDenseGemvRows * 16),
+                       (unsigned)((kDenseGemvRows * (cols + kDenseGemvPad) + cols) * 2), stream, s, x, cols);
+  };
+  if (cols <= 1024) run(dense_gemv_kernel<2>);
+  else if (cols <= 3072) run(dense_gemv_kernel<6>);
+  else run(dense_gemv_kernel<8>);
   return hipGetLastError();
 }
 

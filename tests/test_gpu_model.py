@@ -150,6 +150,31 @@ def test_attention_edges_match_oracle(ctx, heads, kv_heads, head_dim, window, st
         release(model, keep)
 
 
+# One-row projections at the edges of their widths (1,024, 3,072 and 4,096
+# columns in 2, 6 and 8 pieces per thread) and of their 4-row work-groups.
+@pytest.mark.parametrize("hidden,heads,kv_heads,head_dim", [
+    (1056, 3, 3, 18), (1024, 11, 1, 2), (32, 24, 8, 128), (32, 55, 11, 56), (64, 32, 4, 128), (3072, 4, 1, 2),
+])
+def test_one_row_projection_edges_match_oracle(ctx, hidden, heads, kv_heads, head_dim):
+    cfg = dict(vocab=61, hidden=hidden, layers=2, heads=heads, kv_heads=kv_heads, head_dim=head_dim, sliding_window=8,
+               context_cap=16, rms_norm_eps=1e-5, **ROPE_20B)
+    w = synth.model_weights(cfg, synth.numpy_normal(np.random.default_rng(9)))
+    hosts = [O.synthetic_layer(9, i, experts=4, hidden=hidden, intermediate=32, top_k=2) for i in range(cfg["layers"])]
+    for L, h in zip(w["layers"], hosts):
+        L["moe_host"] = h
+    model, keep = build(ctx, cfg, w, hosts)
+    try:
+        oracle = O.ModelHost(cfg, w["embedding"], w["final_norm"], w["lm_head"], w["layers"])
+        prompt = np.array([5], np.uint32)
+        st, want_tokens, want_logits = O.model_generate(oracle, prompt, 3, threads=8)
+        assert st == O.OK
+        assert_bits(model.prefill(prompt), want_logits[0])
+        for k in range(3):
+            assert_bits(model.decode(want_tokens[k]), want_logits[k + 1])
+    finally:
+        release(model, keep)
+
+
 def test_small_model_failed_step_changes_nothing(tiny):
     cfg, model, oracle = tiny
     _, want_tokens, want_logits = O.model_generate(oracle, PROMPT, 2, threads=4)
