@@ -3367,10 +3367,18 @@ __global__ __launch_bounds__(RouteGemvGeom::kThreads, 4) void route_gemv_kernel(
 // whole block at 40 rows of the 20B shape takes 323 us, 2,166 us with the
 // kernel before it, which read every input value from global memory for each
 // weight row; 1 row 56 / 211 us, 300 rows 1,522 / 11,340 us.
+//
+// Rows too long for LDS (K above 10,160) go through it in pieces of kExactPiece
+// values, the accumulators kept, so that a pass holds 8 routes and a CU three
+// work-groups whatever K is; passes of the 4 routes or the one that fit whole
+// left no K above 81,392. Whole calls, 8 experts, top-2, intermediate 1,024, 32
+// rows: hidden 16,384 631 us by whole rows, 596 us by pieces; 20,480 1,312 / 638;
+// 40,960 3,260 / 1,485; 4 rows of 16,384 199 / 203.
 
 constexpr int kExactRows = 64;    // weight rows per work-group
 constexpr int kExactRoutes = 8;   // routes per pass
 constexpr int kExactTN = kExactRows / 32;
+constexpr int kExactPiece = 2944;  // values of a piece of rows too long for LDS (a multiple of 128; 3 work-groups per CU)
 constexpr int kExactFold = 4;     // routes folded at once
 constexpr int kExactPad = 8;      // dwords after each input row in LDS
 
@@ -3429,35 +3437,42 @@ __device__ __forceinline__ void exact_group(float (&acc)[kExactTN][T][2], const 
   }
 }
 
-template <int MODE, int T>
-__device__ __forceinline__ void exact_pass(const GemmArgs& a, int expert, int start, int count, uint32_t* xs, float* fold) {
+// WHOLE: a piece is a whole input row.
+template <int MODE, int T, bool WHOLE>
+__device__ __forceinline__ void exact_pass(const GemmArgs& a, int expert, int start, int count, int piece, uint32_t* xs,
+                                           float* fold) {
   const int tid = threadIdx.x, p = tid & 7, group = tid >> 3;
   const int rows = (int)a.w.rows, B = (int)a.w.blocks, K = B * kBlock, tiles = (int)a.w.tiles;
-  const int nq4 = (B + 3) >> 2, xstride = K / 2 + kExactPad;
+  const int nq4 = (B + 3) >> 2, xstride = (WHOLE ? K : piece) / 2 + kExactPad;
   const int row0 = (int)blockIdx.x * kExactRows;
-  // The pass's input rows (past the item: its last one again).
-  int inexact = a.fast_ok ? 0 : 1;
-  for (int t = tid >> 5; t < T; t += 8) {
-    const int r = start + min(t, count - 1);
-    const uint16_t* src = a.xin + (size_t)(MODE == kGateUp ? a.route_tok[r] : r) * K;
-    const bool aligned = (reinterpret_cast<uintptr_t>(a.xin) & 15) == 0;  // the caller's rows may not be
-#pragma unroll 4
-    for (int c = tid & 31; c < K / 8; c += 32) {
-      u32x4 d;
-      if (aligned) {
-        d = reinterpret_cast<const u32x4*>(src)[c];
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) d[q] = (uint32_t)src[c * 8 + 2 * q] | ((uint32_t)src[c * 8 + 2 * q + 1] << 16);
-      }
-      *reinterpret_cast<u32x4*>(xs + t * xstride + c * 4) = d;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) inexact |= !route_exact_bf16(d[q] & 0xffffu) | !route_exact_bf16(d[q] >> 16);
-    }
-  }
+  int scales = a.fast_ok ? 0 : 1;  // a scale outside kTileFast's range
   if (tid < kExactRows / kTileRows)
-    inexact |= a.w.fast[(size_t)expert * tiles + min(row0 / kTileRows + tid, tiles - 1)] < kTileFast;
-  const bool exact = __syncthreads_or(inexact) == 0;
+    scales |= a.w.fast[(size_t)expert * tiles + min(row0 / kTileRows + tid, tiles - 1)] < kTileFast;
+  // The pass's input rows (past the item: its last one again), values [k0, k0 +
+  // piece); true where every value and scale makes exact products.
+  auto stage = [&](int k0) -> bool {
+    int inexact = scales;
+    const int pieces = (WHOLE ? K : min(piece, K - k0)) / 8;  // of 16 bytes
+    for (int t = tid >> 5; t < T; t += 8) {
+      const int r = start + min(t, count - 1);
+      const uint16_t* src = a.xin + (size_t)(MODE == kGateUp ? a.route_tok[r] : r) * K + k0;
+      const bool aligned = (reinterpret_cast<uintptr_t>(a.xin) & 15) == 0;  // the caller's rows may not be
+#pragma unroll 4
+      for (int c = tid & 31; c < pieces; c += 32) {
+        u32x4 d;
+        if (aligned) {
+          d = reinterpret_cast<const u32x4*>(src)[c];
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) d[q] = (uint32_t)src[c * 8 + 2 * q] | ((uint32_t)src[c * 8 + 2 * q + 1] << 16);
+        }
+        *reinterpret_cast<u32x4*>(xs + t * xstride + c * 4) = d;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) inexact |= !route_exact_bf16(d[q] & 0xffffu) | !route_exact_bf16(d[q] >> 16);
+      }
+    }
+    return __syncthreads_or(inexact) == 0;
+  };
 
   // Weight rows group + 32 n (past the end: the last tile's).
   const __amdgpu_buffer_rsrc_t nib = buffer_rsrc(a.w.nib + (size_t)expert * a.w.nib_stride);
@@ -3480,15 +3495,21 @@ __device__ __forceinline__ void exact_pass(const GemmArgs& a, int expert, int st
   };
   float acc[kExactTN][T][2] = {};
   ExactW cur[kExactTN], next[kExactTN];
-  fetch(0, cur);
 #pragma unroll 1
-  for (int q = 0; q < nq4; ++q) {
-    fetch(min(q + 1, nq4 - 1), next);
-    const int nb = min(4, B - 4 * q);
-    if (exact) exact_group<T, true>(acc, cur, xs + p + q * 64, xstride, nb, byte);
-    else exact_group<T, false>(acc, cur, xs + p + q * 64, xstride, nb, byte);
+  for (int k0 = 0; WHOLE ? k0 == 0 : k0 < K; k0 += WHOLE ? 1 : piece) {  // uniform
+    if (!WHOLE && k0 != 0) __syncthreads();  // every thread is done with the last piece
+    const bool exact = stage(k0);
+    const int q0 = WHOLE ? 0 : k0 / (4 * kBlock), nq = WHOLE ? nq4 : min(q0 + piece / (4 * kBlock), nq4);
+    fetch(q0, cur);
+#pragma unroll 1
+    for (int q = q0; q < nq; ++q) {
+      fetch(min(q + 1, nq4 - 1), next);
+      const int nb = min(4, B - 4 * q);
+      if (exact) exact_group<T, true>(acc, cur, xs + p + (q - q0) * 64, xstride, nb, byte);
+      else exact_group<T, false>(acc, cur, xs + p + (q - q0) * 64, xstride, nb, byte);
 #pragma unroll
-    for (int n = 0; n < kExactTN; ++n) cur[n] = next[n];
+      for (int n = 0; n < kExactTN; ++n) cur[n] = next[n];
+    }
   }
 
   // kExactFold routes at a time: the lane sums [route][row][lane] in LDS, folded
@@ -3538,25 +3559,26 @@ __device__ __forceinline__ void exact_pass(const GemmArgs& a, int expert, int st
   __syncthreads();  // the LDS is free for the next pass
 }
 
-// Dynamic LDS: the input rows; the fold buffers reuse it after the K loop.
-static size_t exact_lds(size_t K, int routes) {
-  const size_t in = (size_t)routes * (K / 2 + kExactPad) * 4;
-  return std::max(in, (size_t)std::min(routes, kExactFold) * kExactRows * 18 * 4);
+// Dynamic LDS: a piece of the input rows; the fold buffers reuse it after the K
+// loop.
+static size_t exact_lds(size_t piece) {
+  const size_t in = (size_t)kExactRoutes * (piece / 2 + kExactPad) * 4;
+  return std::max(in, (size_t)kExactFold * kExactRows * 18 * 4);
 }
 
-template <int MODE>
-__global__ __launch_bounds__(256, 3) void exact_kernel(GemmArgs a, int routes) {
+template <int MODE, bool WHOLE>
+__global__ __launch_bounds__(256, 3) void exact_kernel(GemmArgs a, int piece) {
   extern __shared__ __align__(16) uint32_t s_exact[];
   const int wi = blockIdx.y;
   const int nw = *a.n_work;
   const int4 rec = reinterpret_cast<const int4*>(a.work)[wi];
   if (wi >= nw) return;  // uniform over the work-group
-  for (int t0 = 0; t0 < rec.z; t0 += routes) {  // uniform
-    const int count = min(routes, rec.z - t0);
+  for (int t0 = 0; t0 < rec.z; t0 += kExactRoutes) {  // uniform
+    const int count = min(kExactRoutes, rec.z - t0);
     float* fold = reinterpret_cast<float*>(s_exact);
-    if (count <= 1) exact_pass<MODE, 1>(a, rec.x, rec.y + t0, count, s_exact, fold);
-    else if (count <= 4) exact_pass<MODE, 4>(a, rec.x, rec.y + t0, count, s_exact, fold);
-    else exact_pass<MODE, kExactRoutes>(a, rec.x, rec.y + t0, count, s_exact, fold);
+    if (count <= 1) exact_pass<MODE, 1, WHOLE>(a, rec.x, rec.y + t0, count, piece, s_exact, fold);
+    else if (count <= 4) exact_pass<MODE, 4, WHOLE>(a, rec.x, rec.y + t0, count, piece, s_exact, fold);
+    else exact_pass<MODE, kExactRoutes, WHOLE>(a, rec.x, rec.y + t0, count, piece, s_exact, fold);
   }
 }
 
@@ -4125,13 +4147,16 @@ hipError_t launch_down_combine(const GemmArgs& d, const float* weights, int top_
 
 hipError_t launch_exact(GemmMode mode, const GemmArgs& a, int grid_work, hipStream_t stream) {
   const dim3 grid((unsigned)((a.w.rows + kExactRows - 1) / kExactRows), (unsigned)grid_work);
-  // Routes per pass: 8, or as many as the LDS holds (K > 10,000 or so).
-  const size_t K = a.w.blocks * kBlock, limit = 160 * 1024 - 1024;
-  const int routes = exact_lds(K, kExactRoutes) <= limit ? kExactRoutes : exact_lds(K, 4) <= limit ? 4 : 1;
-  const unsigned lds = (unsigned)exact_lds(K, routes);
-  if (lds > limit) return hipErrorInvalidValue;
-  if (mode == kGateUp) hipLaunchKernelGGL(exact_kernel<kGateUp>, grid, dim3(256), lds, stream, a, routes);
-  else if (mode == kDown) hipLaunchKernelGGL(exact_kernel<kDown>, grid, dim3(256), lds, stream, a, routes);
+  // The input rows whole while 8 of them fit in LDS (K up to 10,160), else by
+  // pieces, so any K is taken.
+  const size_t K = a.w.blocks * kBlock;
+  const bool whole = exact_lds(K) <= 160 * 1024 - 1024;
+  const int piece = whole ? (int)K : kExactPiece;
+  const auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), (unsigned)exact_lds(piece), stream, a, piece);
+  };
+  if (mode == kGateUp) whole ? run(exact_kernel<kGateUp, true>) : run(exact_kernel<kGateUp, false>);
+  else if (mode == kDown) whole ? run(exact_kernel<kDown, true>) : run(exact_kernel<kDown, false>);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }

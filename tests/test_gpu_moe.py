@@ -144,6 +144,25 @@ def test_exact_bf16_passes_and_inexact_products(ctx, m, shrink, scales):
     close(layer)
 
 
+@pytest.mark.parametrize("hidden,inter", [(10144, 32), (10176, 32), (32, 10176), (81408, 32), (32, 81408)])
+def test_exact_bf16_rows_longer_than_lds(ctx, hidden, inter):
+    """Input rows at the longest that exact_kernel holds whole (10,160 values),
+    past it, and past the longest single row that fits in LDS (81,392), which
+    go through LDS by pieces: passes of 8 routes and of 1, with one value whose
+    products round in the second piece only."""
+    host = O.synthetic_layer(47, 0, experts=2, hidden=hidden, intermediate=inter, top_k=2)
+    x = O.gen_hidden(47, 900, 9, hidden)
+    x[3, 3000 % hidden] = synth.bf16_bits(np.array([2.0 ** -100], np.float32))[0]
+    want = O.moe_batch(host, x, trace=True, projection=G.PROJECTION_EXACT_BF16)
+    assert want["status"] == O.OK
+    layer = gpu_layer(ctx, host, G.PROJECTION_EXACT_BF16)
+    got = layer.forward(x, trace=True)
+    assert_moe_equal(got, want)
+    assert_traces_equal(got, want)
+    assert not G.circuit_is_open()
+    close(layer)
+
+
 def test_unknown_projection_is_rejected(ctx):
     host = O.synthetic_layer(3, 0, experts=2, hidden=64, intermediate=32, top_k=1)
     with pytest.raises(G.GossmxError) as e:
