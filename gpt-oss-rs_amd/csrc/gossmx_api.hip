@@ -564,6 +564,7 @@ hipStream_t context_stream(const gossmx_ctx* ctx) { return ctx->stream; }
 int run_time_result(gossmx_ctx* ctx, int status) { return projection_result(ctx, status); }
 const int* context_error_flags(const gossmx_ctx* ctx) { return ctx->err; }
 int error_flags_result(gossmx_ctx* ctx, int flags) { return flags == 0 ? GOSSMX_OK : device_flags_fail(ctx, flags); }
+int context_errors(gossmx_ctx* ctx) { return check_device_errors(ctx); }
 
 void count_transfer(int direction, size_t bytes) {
   if (direction >= 0 && direction < 3) g_stats.transfer[direction].fetch_add(bytes, std::memory_order_relaxed);

@@ -370,7 +370,8 @@ size_t out_bytes(const gossmx_model_config& c) { return c.layers * sizeof(gossmx
 
 // Enqueues one layer-major step over the m rows whose embeddings are in
 // host_in, and the copy of its marks and the last row's logits to host_out.
-int enqueue_step(gossmx_model* M, size_t m, const StepRows& R, hipStream_t stream) {
+// *enqueued counts the layers whose MoE call was enqueued.
+int enqueue_step(gossmx_model* M, size_t m, const StepRows& R, hipStream_t stream, size_t* enqueued) {
   const gossmx_model_config& c = M->cfg;
   DenseDevice& D = M->dev;
   const size_t H = c.hidden, QW = c.heads * c.head_dim, KW = c.kv_heads * c.head_dim, n = m * H;
@@ -435,6 +436,7 @@ int enqueue_step(gossmx_model* M, size_t m, const StepRows& R, hipStream_t strea
     const int st = gossmx_moe_forward_residual(M->ctx, M->layers[li].moe, &io, L.post_norm, c.rms_norm_eps, next);
     (void)gossmx_profile_tag(M->ctx, -1, GOSSMX_PHASE_UNKNOWN);
     if (st != GOSSMX_OK) return st;
+    ++*enqueued;
     std::swap(hidden, next);
   }
   // Final norm and lm_head for the last row (the only row whose logits are required).
@@ -484,10 +486,14 @@ int gpu_step(gossmx_model* M, const uint32_t* tokens, size_t m, double* moe) {
     if (int st = grow_ring(M, kv, M->position, m, stream)) return st;
   for (size_t r = 0; r < m; ++r)
     std::memcpy(D.host_in + r * H * 2, M->embedding + (size_t)tokens[r] * H, H * 2);
-  const int st = enqueue_step(M, m, R, stream);
+  size_t enqueued = 0;
+  const int st = enqueue_step(M, m, R, stream, &enqueued);
   if (st != GOSSMX_OK) {
     (void)hipStreamSynchronize(stream);  // the staging buffers' copies end before the next step reuses them
-    return st;
+    // An earlier layer may have raised the error flags: its error comes first,
+    // and the flags are not left for the next call.
+    const int raised = enqueued ? gossmx::context_errors(M->ctx) : GOSSMX_OK;
+    return raised != GOSSMX_OK ? raised : st;
   }
   DENSE_HIP(hipStreamSynchronize(stream), "model step");
   const gossmx::ModelMark* marks = reinterpret_cast<const gossmx::ModelMark*>(D.host_out);

@@ -328,9 +328,10 @@ const gossmx_moe_config* layer_config(const gossmx_layer* layer);
 int context_device(const gossmx_ctx* ctx);
 hipStream_t context_stream(const gossmx_ctx* ctx);
 // The context's device error flags, and the status of a value read from them
-// (cleared when not zero).
+// (cleared when not zero), or of the flags as they are (synchronizes).
 const int* context_error_flags(const gossmx_ctx* ctx);
 int error_flags_result(gossmx_ctx* ctx, int flags);
+int context_errors(gossmx_ctx* ctx);
 // A GPU round trip's status: GOSSMX_ERR_DEVICE or GOSSMX_ERR_OUT_OF_MEMORY
 // drains the context's stream and opens the process-wide circuit breaker.
 int run_time_result(gossmx_ctx* ctx, int status);

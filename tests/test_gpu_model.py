@@ -232,6 +232,42 @@ def test_small_model_device_flag_failure_opens_the_breaker(ctx, tiny):
     assert_bits(model.decode(want_tokens[0]), want_logits[1])
 
 
+def test_refused_layer_leaves_no_error_flags(ctx):
+    # Layer 1 refuses a step of 1,024 rows (its down input would pass the 32-bit
+    # offsets) after layer 0's call was enqueued. Where layer 0 raised the
+    # device error flags, the step reports them, as the oracle does; and the
+    # next step finds neither the flags nor the rows of the failed one.
+    cfg = dict(vocab=64, hidden=32, layers=2, heads=2, kv_heads=1, head_dim=4, sliding_window=4, context_cap=1100,
+               rms_norm_eps=1e-5, **ROPE_20B)
+    w = synth.model_weights(cfg, synth.numpy_normal(np.random.default_rng(10)))
+    w["embedding"][63] = 0x7F80  # infinities: layer 0's router logits are not finite
+    hosts = [O.synthetic_layer(10, 0, experts=4, hidden=32, intermediate=32, top_k=2),
+             O.synthetic_layer(10, 1, experts=4, hidden=32, intermediate=131072, top_k=4)]
+    for L, h in zip(w["layers"], hosts):
+        L["moe_host"] = h
+    model, keep = build(ctx, cfg, w, hosts)
+    try:
+        oracle = O.ModelHost(cfg, w["embedding"], w["final_norm"], w["lm_head"], w["layers"])
+        st, want_tokens, want_logits = O.model_generate(oracle, PROMPT % 63, 1, threads=8)
+        assert st == O.OK and want_tokens[0] != 63
+        assert_bits(model.prefill(PROMPT % 63), want_logits[0])
+        rows = np.arange(1024, dtype=np.uint32) % 63
+        before = [model.cache(i) for i in range(2)]
+        for bad, status in ((None, G.ERR_UNSUPPORTED), (700, G.ERR_NON_FINITE_LOGITS)):
+            if bad is not None:
+                rows[bad] = 63
+                assert O.model_generate(oracle, rows[bad:], 0, threads=8)[0] == O.NON_FINITE_LOGITS
+            with pytest.raises(G.GossmxError) as e:
+                model.append(rows)
+            assert e.value.status == status
+            ctx.synchronize()  # would report flags that were left
+            assert not G.circuit_is_open()
+            assert model.position == PROMPT.size and [model.cache(i) for i in range(2)] == before
+        assert_bits(model.decode(want_tokens[0]), want_logits[1])
+    finally:
+        release(model, keep)
+
+
 def test_small_model_profile_records_carry_layer_and_phase(ctx, tiny):
     # The model step tags its MoE calls with the layer index and the phase
     # (CpuExecutionProfileRecord's layer and phase, cpu_profile.rs:121-150);
