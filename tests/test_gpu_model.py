@@ -268,6 +268,81 @@ def test_refused_layer_leaves_no_error_flags(ctx):
         release(model, keep)
 
 
+def test_failed_step_on_wrapped_rings_changes_nothing(ctx):
+    # The sliding layer's ring (256 slots) has wrapped when a step writes its 30
+    # rows there and fails: one row's embedding is infinite, so that the logits
+    # are not finite. The rows of the window stay as they were.
+    cfg = dict(TINY, sliding_window=100, context_cap=400)
+    w = synth.model_weights(cfg, synth.numpy_normal(np.random.default_rng(11)))
+    w["embedding"][299] = 0x7F80
+    hosts = [O.synthetic_layer(11, i, experts=4, hidden=64, intermediate=32, top_k=2) for i in range(2)]
+    for L, h in zip(w["layers"], hosts):
+        L["moe_host"] = h
+    model, keep = build(ctx, cfg, w, hosts)
+    try:
+        oracle = O.ModelHost(cfg, w["embedding"], w["final_norm"], w["lm_head"], w["layers"])
+        prompt = ((np.arange(330, dtype=np.uint32) * 2654435761) >> 7) % 299
+        st, want_tokens, want_logits = O.model_generate(oracle, prompt, 2, threads=8)
+        assert st == O.OK and 299 not in want_tokens
+        for lo in range(0, 300, 50):
+            model.append(prompt[lo:lo + 50])
+        before = [model.cache(i) for i in range(2)]
+        assert before == [(100, 200), (300, 0)]
+        for at in (0, 29):
+            rows = prompt[:30].copy()
+            rows[at] = 299
+            with pytest.raises(G.GossmxError) as e:
+                model.append(rows)
+            assert e.value.status == G.ERR_NON_FINITE_LOGITS
+            assert model.position == 300 and [model.cache(i) for i in range(2)] == before
+        assert_bits(model.append(prompt[300:]), want_logits[0])
+        for k in range(2):
+            assert_bits(model.decode(want_tokens[k]), want_logits[k + 1])
+    finally:
+        release(model, keep)
+
+
+# Infinities and NaN in attention's operands: a head whose scores are all -inf
+# (its sink takes the whole softmax), sinks of -inf and so large that no score
+# counts, and values that make the step's logits non-finite, as in the oracle.
+@pytest.mark.parametrize("window,change,finite", [
+    (1, {"q_bias": 1e25, "k_bias": -1e25}, True),
+    (4, {"sinks": -np.inf}, True),
+    (4, {"sinks": 1e30}, True),
+    (4, {"sinks": np.inf}, False),
+    (4, {"sinks": np.nan}, False),
+    (1, {"q_bias": 1e25, "k_bias": 1e25}, False),
+    (4, {"q_bias": np.nan}, False),
+    (4, {"k_bias": np.inf}, False),
+    (4, {"v_bias": np.inf}, False),
+])
+def test_attention_special_values_match_oracle(ctx, window, change, finite):
+    cfg = dict(TINY, sliding_window=window)
+    w = synth.model_weights(cfg, synth.numpy_normal(np.random.default_rng(12)))
+    for name, value in change.items():  # head 0 of the first layer, and its kv head
+        n = 1 if name == "sinks" else cfg["head_dim"]
+        w["layers"][0][name] = w["layers"][0][name].copy()
+        w["layers"][0][name][:n] = value
+    hosts = [O.synthetic_layer(12, i, experts=4, hidden=64, intermediate=32, top_k=2) for i in range(2)]
+    for L, h in zip(w["layers"], hosts):
+        L["moe_host"] = h
+    model, keep = build(ctx, cfg, w, hosts)
+    try:
+        oracle = O.ModelHost(cfg, w["embedding"], w["final_norm"], w["lm_head"], w["layers"])
+        st, want_tokens, want_logits = O.model_generate(oracle, PROMPT, 2, threads=4)
+        assert (st == O.OK) == finite
+        if finite:
+            assert_bits(model.prefill(PROMPT), want_logits[0])
+            for k in range(2):
+                assert_bits(model.decode(want_tokens[k]), want_logits[k + 1])
+        else:
+            with pytest.raises(G.GossmxError) as e:
+                model.prefill(PROMPT)
+            assert e.value.status == st
+    finally:
+        release(model, keep)
+
+
 def test_small_model_profile_records_carry_layer_and_phase(ctx, tiny):
     # The model step tags its MoE calls with the layer index and the phase
     # (CpuExecutionProfileRecord's layer and phase, cpu_profile.rs:121-150);

@@ -362,6 +362,68 @@ def test_router_tiles_bit_exact(ctx, experts, hidden, m, norm, shrink):
     close(layer)
 
 
+def forward_unaligned(ctx, layer, x, logits=None):
+    """forward on device rows that start two bytes past a 16-byte boundary."""
+    m, E, K, H = x.shape[0], layer.experts, layer.top_k, layer.hidden
+    res = {"router_logits": np.empty((m, E), np.float32), "selected": np.empty((m, K), np.uint32),
+           "routing_weights": np.empty((m, K), np.float32), "output": np.empty((m, H), np.float32),
+           "route_order": np.empty(m * K, np.uint32)}
+    dev = {k: ctx.malloc(v.nbytes) for k, v in res.items()}
+    dx = ctx.malloc(x.nbytes + 16)
+    dl = ctx.malloc(logits.nbytes) if logits is not None else None
+    try:
+        ctx.h2d(dx, np.concatenate([np.zeros(1, np.uint16), x.ravel()]))
+        if dl is not None:
+            ctx.h2d(dl, logits)
+        layer.forward_device(dx + 2, m, injected_logits=dl, **dev)
+        ctx.synchronize()
+        for k, v in res.items():
+            ctx.d2h(v, dev[k])
+    finally:
+        for p in [dx, dl, *dev.values()]:
+            if p is not None:
+                ctx.free(p)
+    return res
+
+
+@pytest.mark.parametrize("projection,hidden,m,inject", [
+    (G.PROJECTION_RESIDUAL_Q8, 96, 5, False),     # f16 codes, 8-row items
+    (G.PROJECTION_Q8, 2880, 37, False),           # 16-row items, two K chunks of the row's dots
+    (G.PROJECTION_RESIDUAL_Q8, 96, 400, False),   # digit records, 32-row items
+    (G.PROJECTION_Q8, 160, 401, False),
+    (G.PROJECTION_RESIDUAL_Q8, 96, 400, True),    # the selection kernel's quantization
+    (G.PROJECTION_EXACT_BF16, 160, 9, False),     # exact_kernel's element-wise row loads
+    (G.PROJECTION_EXACT_BF16, 10176, 5, False),   # ... in pieces
+])
+def test_unaligned_device_rows_bit_exact(ctx, projection, hidden, m, inject):
+    """Rows that are not 16-byte aligned take the row-by-row router
+    (route_kernel) and the exact projection's element-wise loads."""
+    host = O.synthetic_layer(53, 0, experts=32, hidden=hidden, intermediate=64, top_k=4)
+    x = O.gen_hidden(53, 1000 + m, m, hidden)
+    logits = None
+    if inject:
+        logits = O.bf16_round_array(np.random.default_rng(m).standard_normal((m, 32)).astype(np.float32))
+    want = O.moe_batch(host, x, injected_logits=logits, projection=projection)
+    assert want["status"] == O.OK
+    layer = gpu_layer(ctx, host, projection)
+    assert_moe_equal(forward_unaligned(ctx, layer, x, logits), want)
+    close(layer)
+
+
+@pytest.mark.parametrize("projection,m", [(G.PROJECTION_RESIDUAL_Q8, 3), (G.PROJECTION_RESIDUAL_Q8, 37),
+                                          (G.PROJECTION_Q8, 400)])
+def test_hidden_past_the_tiled_router_bit_exact(ctx, projection, m):
+    """A hidden size above 8,192: the row-by-row router, with f16 codes and with
+    the digit records of 32-row items."""
+    host = O.synthetic_layer(59, 0, experts=32, hidden=8224, intermediate=32, top_k=4)
+    x = O.gen_hidden(59, 1100 + m, m, 8224)
+    want = O.moe_batch(host, x, projection=projection)
+    assert want["status"] == O.OK
+    layer = gpu_layer(ctx, host, projection)
+    assert_moe_equal(layer.forward(x), want)
+    close(layer)
+
+
 @pytest.fixture(scope="module")
 def layer120b(ctx):
     host = O.synthetic_layer(120, 0, experts=128)
