@@ -845,7 +845,7 @@ constexpr size_t kWideRows = 16, kWideRoutes = 1280, kWideRoutesQ8 = 512;
 static int gemm_chunk(size_t m, size_t routes, size_t experts, bool residual) {
   if (m <= (size_t)kSmallChunk) return kSmallChunk;
   const size_t least = residual && experts > 1 ? kWideRoutes : kWideRoutesQ8;
-  return routes >= std::max(least, kWideRows * experts) ? kHugeChunk : kChunk;
+  return routes >= std::max(least, kWideRows * experts) ? kWideChunk : kChunk;
 }
 
 // Batches of at most kTinyMaxRows rows on weights of at most kTinyMaxBlocks
@@ -886,7 +886,7 @@ static int matmul_impl(gossmx_ctx* ctx, const gossmx_matmul_problem* p) {
   const bool gemv = use_gemv(m, B, p->activation_kind == GOSSMX_ACT_RESIDUAL_Q8);
   const int chunk = gemm_chunk(m, m, 1, p->activation_kind == GOSSMX_ACT_RESIDUAL_Q8);
   ActBuffers act{static_cast<_Float16*>(ctx->act1v.p), static_cast<float*>(ctx->act1s.p),
-                 !gemv && chunk == kHugeChunk ? 1 : 0};
+                 !gemv && chunk == kWideChunk ? 1 : 0};
   HIP_TRY(launch_prep_records(rec, p->activation_kind, m, B, p->row_stride, act, ctx->err, ctx->stream),
           "prepare activations");
   const float* bias = p->bias;
@@ -1067,7 +1067,7 @@ static int moe_forward_impl(gossmx_ctx* ctx, const gossmx_layer* L, const gossmx
       (s = take(ctx, arena, ctx->act2s, R * B2 * 8 + kActSlack, &act2.s)) ||
       (s = take(ctx, arena, ctx->y, R * H * 2, &ybuf)))
     return s;
-  act1.digits = act2.digits = proj != GOSSMX_PROJECTION_EXACT_BF16 && chunk == kHugeChunk ? 1 : 0;
+  act1.digits = act2.digits = proj != GOSSMX_PROJECTION_EXACT_BF16 && chunk == kWideChunk ? 1 : 0;
   // Batches whose logits fit one work-group take the fused selection +
   // dispatch kernel; larger ones a selection kernel with per-work-group
   // expert counts and a placement kernel. The router projection (when the

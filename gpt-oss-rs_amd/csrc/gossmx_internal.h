@@ -14,7 +14,7 @@ constexpr int kTileRows = 16;   // rows per MFMA tile (one wave)
 constexpr int kWgRows = 64;     // gate_up rows (32 gate/up pairs) per 32-value block of the down input
 constexpr int kChunk = 16;      // activation rows per GEMM work item (batches of more than kSmallChunk rows)
 constexpr int kSmallChunk = 8;  // activation rows per work item for batches of at most 8 rows
-constexpr int kHugeChunk = 32;  // activation rows per work item where experts hold many rows (gemm_chunk)
+constexpr int kWideChunk = 32;  // activation rows per work item where experts hold many rows (gemm_chunk)
 constexpr int kChunkMax = 32;
 // Small-batch GEMV (gemv_kernel): batches of at most kTinyMaxRows rows whose
 // blocks per row are at most kTinyMaxBlocks (the activation image of the
@@ -140,7 +140,7 @@ struct DispatchArgs {
   int* route_slot;      // [routes]
   int* work;            // [max_work][4] (expert, first grouped route, rows, 0): one record per item
   int* n_work;
-  int chunk;            // rows per work item: kSmallChunk, kChunk or kHugeChunk (by batch size)
+  int chunk;            // rows per work item: kSmallChunk, kChunk or kWideChunk (gemm_chunk)
 };
 
 // Batches whose logits fit one work-group's LDS take the fused selection +
@@ -178,7 +178,7 @@ hipError_t launch_select_dispatch(const RouteArgs& r, const DispatchArgs& d, int
 // quantization of m <= kFusedRouteRows rows in one launch. `counter`: a
 // device int that is 0 before the launch; the launch leaves it 0.
 hipError_t launch_route_select(const RouteArgs& r, const DispatchArgs& d, int* counter, hipStream_t stream);
-// chunk: rows per work item (kSmallChunk, kChunk or kHugeChunk), selecting
+// chunk: rows per work item (kSmallChunk, kChunk or kWideChunk), selecting
 // the kernel's geometry; it must match the chunk the dispatch used.
 // start/stop (nullable): events the launch itself records around the kernel.
 hipError_t launch_gemm(GemmMode mode, const GemmArgs& a, int chunk, int grid_work, hipStream_t stream,

@@ -265,8 +265,9 @@ __device__ __forceinline__ void q8_scales_n(const float (&mx)[N], int l32, float
 // residual_q8_store for N blocks per half wave at once (block i is item
 // hw + i * stride: activation row first_row + item / per_row, block
 // first_blk + item % per_row); blocks with live[i] false are computed on
-// zeros and not stored. The same operations as residual_q8_store per block.
-template <int N, bool RESIDUAL, bool DIGITS = false>
+// zeros and not stored. The same operations as residual_q8_store per block, with
+// f16 codes.
+template <int N, bool RESIDUAL>
 __device__ __forceinline__ void residual_q8_store_n(const float (&v)[N], const bool (&live)[N], int l32, int hw,
                                                     int stride, int per_row, size_t first_row, int blocks,
                                                     int first_blk, ActBuffers act) {
@@ -307,15 +308,9 @@ __device__ __forceinline__ void residual_q8_store_n(const float (&v)[N], const b
     const int item = hw + i * stride;
     const size_t row = first_row + item / per_row;
     const int blk = first_blk + item % per_row;
-    if (DIGITS) {
-      uint8_t* rec = reinterpret_cast<uint8_t*>(act.v) + (row * blocks + blk) * kDigitRecord;
-      store_digits(rec, q[i], l32);
-      if (RESIDUAL) store_digits(rec + kDigitRecord / 2, rq[i], l32);
-    } else {
-      _Float16* dst = act.v + ((row * blocks + blk) * 2) * kBlock;
-      dst[l32] = (_Float16)q[i];
-      dst[kBlock + l32] = (_Float16)rq[i];
-    }
+    _Float16* dst = act.v + ((row * blocks + blk) * 2) * kBlock;
+    dst[l32] = (_Float16)q[i];
+    dst[kBlock + l32] = (_Float16)rq[i];
     if (l32 == 0) {
       float2 sc;
       sc.x = s[i];
@@ -1236,15 +1231,17 @@ typedef __attribute__((address_space(3))) void* lds_ptr;
 // work items of NTOK activation rows (NTOK / 8 MFMA token groups), K steps of
 // GROUPS 4-block groups, WAVES waves per work-group, and MIN_WAVES waves per
 // SIMD that the register budget must allow.
-//  GemmBig (2 tiles, 16 rows, 4 blocks, 4 waves) serves batches of 9..511
-//    rows: 96 VGPRs and 27.7 KB of LDS give 5 work-groups per CU, 5 waves per
-//    SIMD to hide the LDS and MFMA latency of the ordered chain.
+//  GemmBig (2 tiles, 16 rows, 4 blocks, 4 waves) serves batches of more than 8
+//    rows whose experts hold too few for gemm_wide_kernel (gemm_chunk, by routes
+//    and experts: up to 319 rows with 32 experts, top-4, residual-Q8, up to 511
+//    with 128): 90 VGPRs and 27.7 KB of LDS give 5 work-groups per CU, 5 waves
+//    per SIMD to hide the LDS and MFMA latency of the ordered chain.
 //  GemmSmall (1 tile, 8 rows, 8 blocks, 4 waves) serves batches of at most 8
 //    rows, whose work items are one expert each and whose time is the weight
-//    stream's latency: 64-row work-groups (four times the big geometry's
-//    count per expert), 73 VGPRs, 5 work-groups per CU.
+//    stream's latency: 64-row work-groups (twice the big geometry's count per
+//    expert), 70 VGPRs, 5 work-groups per CU.
 // Batches whose experts hold many rows run gemm_wide_kernel instead.
-template <int TILES, int NTOK, int GROUPS, int WAVES = 8, int MIN_WAVES = 4, int WLEAD = 2>
+template <int TILES, int NTOK, int GROUPS, int WAVES, int MIN_WAVES>
 struct GemmCfg {
   static constexpr int kWaves = WAVES;                    // waves per work-group
   static constexpr int kThreads = 64 * WAVES;
@@ -1263,20 +1260,16 @@ struct GemmCfg {
   // scale dword) per tile; activations kCodeDma code pieces + 1 scale dword.
   static constexpr int kLoadsW = 2 * GROUPS * TILES;
   static constexpr int kLoadsD = kCodeDma + 1;
-  // Steps by which the weight requests lead their use (1 or 2; the DMA leads
-  // by 2).
-  static constexpr int kWLead = WLEAD;
   // s_waitcnt immediate for "the DMA and the weights of step q have landed":
-  // issued after them are D(q+1) and, with a two-step lead, W(q+1) (see
-  // k_loop). expcnt and lgkmcnt are not waited on.
-  static constexpr int kWaitVm = (WLEAD == 2 ? kLoadsW : 0) + kLoadsD;
+  // issued after them are D(q+1) and W(q+1) (see k_loop). expcnt and lgkmcnt are
+  // not waited on.
+  static constexpr int kWaitVm = kLoadsW + kLoadsD;
   static constexpr int kWaitDma = (kWaitVm & 15) | ((kWaitVm >> 4) << 14) | (7 << 4) | (15 << 8);
   static_assert(kSlotBytes == kCodeDma * 16 * kThreads, "code DMA covers a slot exactly");
   static_assert(kStep * NTOK * 2 <= kSclSlot, "one dword DMA per lane covers a step's scales");
   static_assert(NTOK % 8 == 0 && NTOK <= kChunkMax, "token groups of 8");
   static_assert(kGemmRows % 64 == 0, "a work-group's gate_up rows make whole 32-value down-input blocks");
   static_assert(kWaitVm < 64, "vmcnt field");
-  static_assert(WLEAD == 1 || WLEAD == 2, "weight lead");
   static_assert((kStep - 1) * 2 * kBlock * 2 <= (int)kActSlack, "a last partial step reads inside the slack");
 };
 using GemmBig = GemmCfg<2, 16, 1, 4, 5>;
@@ -1689,17 +1682,13 @@ __device__ __forceinline__ void step_update(const KLoop<C>& k, Acc<C>& tot, cons
 }
 
 // The K loop. Vector-memory issue order per wave, fixed so that one
-// immediate wait covers every step. With a two-step weight lead:
+// immediate wait covers every step:
 //   prologue W(0) D(0) W(1) D(1); step q: wait(D(q), W(q)) barrier
 //   D(q+2) compute(q) W(q+2);
 // at step q's wait the requests after D(q) and W(q) are D(q+1) and W(q+1)
-// = kWaitVm instructions. With a one-step lead:
-//   prologue W(0) D(0) D(1); step q: wait(D(q), W(q)) barrier
-//   W(q+1) D(q+2) compute(q);
-// at step q's wait only D(q+1) follows W(q). A three-step weight lead queued
-// more requests ahead of each step's own and ran 1% slower on decode batches;
-// prefill, with four token groups of compute per step, runs 1-2% faster with
-// a one-step lead, decode 0.5% slower.
+// = kWaitVm instructions. Decode batches ran 1% slower with weights requested
+// three steps ahead (more requests ahead of each step's own) and 0.5% slower
+// with one step.
 template <class C, bool RESIDUAL, int NTG, bool FAST>
 __device__ __forceinline__ void k_loop(const KLoop<C>& k, Acc<C>& tot, char* c0, char* c1, char* c2, float* s0,
                                        float* s1, float* s2) {
@@ -1709,31 +1698,29 @@ __device__ __forceinline__ void k_loop(const KLoop<C>& k, Acc<C>& tot, char* c0,
   __builtin_amdgcn_sched_barrier(0);
   issue_dma<C>(k, 0, c0, s0);
   __builtin_amdgcn_sched_barrier(0);
-  if (C::kWLead == 2) w1 = load_wstep(k, 1);
+  w1 = load_wstep(k, 1);
   __builtin_amdgcn_sched_barrier(0);
   issue_dma<C>(k, 1, c1, s1);
   __builtin_amdgcn_sched_barrier(0);
-#define GOSSMX_STEP(QV, SLOT, CODES, SCL, NCODES, NSCL, NEXT1, NEXT2)                               \
+#define GOSSMX_STEP(QV, SLOT, CODES, SCL, NCODES, NSCL, NEXT)                                       \
   {                                                                                                  \
     const int q = (QV);                                                                              \
     __builtin_amdgcn_sched_barrier(0);                                                               \
     __builtin_amdgcn_s_waitcnt(C::kWaitDma); /* this wave's DMA and weights for step q have landed */\
     __builtin_amdgcn_s_barrier();         /* ... and every other wave's; the slot of q-1 is free */  \
     __builtin_amdgcn_sched_barrier(0);                                                               \
-    if (C::kWLead == 1) NEXT1 = load_wstep(k, q + 1);                                                \
-    __builtin_amdgcn_sched_barrier(0);                                                               \
     issue_dma<C>(k, q + 2, NCODES, NSCL);                                                            \
     __builtin_amdgcn_sched_barrier(0);                                                               \
     if (k.wave_ok && q < k.nsteps) step_update<C, RESIDUAL, NTG, FAST>(k, tot, CODES, SCL, SLOT, q); \
     __builtin_amdgcn_sched_barrier(0);                                                               \
-    if (C::kWLead == 2) NEXT2 = load_wstep(k, q + 2);                                                \
+    NEXT = load_wstep(k, q + 2);                                                                     \
     __builtin_amdgcn_sched_barrier(0);                                                               \
   }
   const int n_pad = (k.nsteps + 2) / 3 * 3;
   for (int q0 = 0; q0 < n_pad; q0 += 3) {
-    GOSSMX_STEP(q0, w0, c0, s0, c2, s2, w1, w2)
-    GOSSMX_STEP(q0 + 1, w1, c1, s1, c0, s0, w2, w0)
-    GOSSMX_STEP(q0 + 2, w2, c2, s2, c1, s1, w0, w1)
+    GOSSMX_STEP(q0, w0, c0, s0, c2, s2, w2)
+    GOSSMX_STEP(q0 + 1, w1, c1, s1, c0, s0, w0)
+    GOSSMX_STEP(q0 + 2, w2, c2, s2, c1, s1, w1)
   }
 #undef GOSSMX_STEP
 }
@@ -1929,7 +1916,7 @@ struct WideCfg {
   static constexpr int kThreads = 64 * kWaves;
   static constexpr int kWgTiles = 2 * kWaves;
   static constexpr int kRows = kTileRows * kWgTiles;   // 256
-  static constexpr int kChunk = kHugeChunk;            // 32 activation rows
+  static constexpr int kChunk = kWideChunk;            // 32 activation rows
   static constexpr int kStep = 4;                      // blocks per step (one group of the v3 layout)
   static constexpr int kSclSlot = kStep * kChunk * 2;  // floats of a step's activation scales
   static constexpr int kWSlot = kWaves * 2048;         // a step's weight groups: two 1 KiB groups per wave
@@ -4071,7 +4058,7 @@ hipError_t launch_gemm(GemmMode mode, const GemmArgs& a, int chunk, int grid_wor
                        hipEvent_t start, hipEvent_t stop) {
   if (chunk == GemmSmall::kChunk) return launch_gemm_cfg<GemmSmall>(mode, a, grid_work, stream, start, stop);
   if (chunk == GemmBig::kChunk) return launch_gemm_cfg<GemmBig>(mode, a, grid_work, stream, start, stop);
-  if (chunk == kHugeChunk) return launch_gemm_wide(mode, a, grid_work, stream, start, stop);
+  if (chunk == kWideChunk) return launch_gemm_wide(mode, a, grid_work, stream, start, stop);
   return hipErrorInvalidValue;
 }
 
