@@ -1882,14 +1882,17 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void gemm_kernel(GemmArg
 // this path). The MFMA takes 32 cycles for 1,024 dots where the f16 form takes
 // 16 for 256, and its FP4 conversions 16 more.
 //
-// Bound: the float chain, four VALU instructions per 64 (weight row, activation
-// row, block) triples; an f32 instruction takes a SIMD four cycles (the MFMAs
-// run beside them), and the counters show the VALU busy for the whole kernel.
-// So everything else is kept out of the VALU: no weight conversion, weights
-// by DMA and transposed by six swaps a step, one scale register per part. At
-// 2,048 rows of the 20B shape gate_up takes 738 us for 348 M VALU instructions
-// (289 M of them the chain; the two-tile f16 kernel before it 881 us for 424 M
-// with its MFMAs), down 362 us (436); 4,096 rows over 128 experts 1,510 and
+// Bound: what a SIMD issues. The float chain is four VALU instructions per 64
+// (weight row, activation row, block) triples, and a SIMD that several waves
+// share runs an f32 multiply or add in two cycles, but no MFMA beside it (a
+// probe ran every mix of the two, in one wave or in different waves, in the sum
+// of their times). Per full step and wave that is 256 chain instructions and 8
+// MFMAs, 512 + 256 cycles, and ten other VALU instructions: no weight conversion,
+// weights by DMA and transposed by six swaps, one scale register per part. At
+// 2,048 rows of the 20B shape gate_up takes 738 us, 1.36 M cycles: 0.56 M of
+// chain, 0.28 M of MFMAs, about 0.13 M of other VALU work (the epilogue most of
+// it); the rest is waiting. The two-tile f16 kernel before it took 881 us with
+// twice the MFMA cycles; down 362 us (436); 4,096 rows over 128 experts 1,510 and
 // 744 us (1,835 and 923); 777 rows in Q8 mode 236 and 126 us (324 and 162).
 // Weights straight into registers, read twice by the two halves of a wave, kept
 // the vector-memory path busy for 72% of the Q8 kernel: 283 us.
@@ -2392,7 +2395,7 @@ __global__ __launch_bounds__(WideCfg::kThreads, 4) void gemm_wide_kernel(GemmArg
 // Bound: VALU instructions (28 per 16 dots' steps at TR = 2, TE = 4) and, for
 // small batches, one memory round trip and the 180-step chain. The small tile
 // (4 rows x 8 experts, the whole K range of its experts staged at once) gives
-// small batches work-groups enough; from kRouteSmallGroups of them on the large
+// small batches work-groups enough; past kRouteSmallGroups of them the large
 // one (8 x 32, experts by chunks of kRouteTileK) does fewer reads per dot.
 // With the norm: 2,048 rows x 32 experts 48 us (282 us by route_kernel, whose
 // work-groups each re-read 16 experts for one row), 256 x 128 40 us (84);
@@ -2400,6 +2403,10 @@ __global__ __launch_bounds__(WideCfg::kThreads, 4) void gemm_wide_kernel(GemmArg
 constexpr int kRouteTileHidden = kNormMaxHidden;
 constexpr int kRouteTileK = 256;        // elements of the large tile's expert chunks
 constexpr int kRoutePad = 8;            // dwords after each LDS row: consecutive rows start 8 banks apart
+// Small against large tiles, 2,880 values, us without / with the norm: 32 experts
+// 512 rows 20 / 30 and 38 / 43, 1,024 rows 32 / 51 and 38 / 42, 1,536 rows 46 / 73
+// and 40 / 43; 128 experts 256 rows 24 / 37 and 28 / 33, 384 rows 33 / 52 and 29 /
+// 33. They cross at about 1,250 groups without the norm and 850 with it.
 constexpr int kRouteSmallGroups = 1024;
 constexpr int kRouteQuantShares = 4;    // quantization work-groups per small row tile
 
@@ -3694,9 +3701,9 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* y, const f
 
 // The f16 operand: a thread moves 8 codes of one part (two dwords in, 16 bytes
 // out; records and their codes are 4-byte aligned). Q8 records leave zeros in
-// part 1. At 129 rows of 90 blocks the
-// whole matmul call takes 26.8 us; 27.2 us with 32 threads per record, two bytes
-// in and four out each.
+// part 1. At 129 rows of 90 blocks the whole matmul call takes 26.9 us, 27.0 with
+// 32 threads per record, two bytes in and four out each: no difference past the
+// noise (27.2 with the digit operand's branch in the same kernel).
 __global__ __launch_bounds__(256) void prep_records_kernel(const uint8_t* rec, int kind, int m, int blocks,
                                                           size_t row_stride, ActBuffers act) {
   const size_t it = (size_t)blockIdx.x * 256 + threadIdx.x;
