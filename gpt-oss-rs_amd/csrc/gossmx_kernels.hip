@@ -174,6 +174,15 @@ __device__ __forceinline__ float half_wave_max(float m) {
 // in three instructions.
 __device__ __forceinline__ float round_half_away(float x) { return truncf(x + copysignf(0x1.fffffep-2f, x)); }
 
+// v * inverse of quantize_q8_block, as its code: the inverse of a scale below
+// 2^-128 is infinite, and there a zero's product is NaN, which Rust's `as i8`
+// makes 0. v_mul_legacy_f32 is the same product but 0 for a zero operand.
+__device__ __forceinline__ float q8_product(float v, float inv) {
+  float r;
+  asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(v), "v"(inv));
+  return r;
+}
+
 // quantize_q8_block (lib.rs:1051-1065) for the 32 values held by a 32-lane
 // half wave (lane l32 holds value l32): scale = max|v| / 127, inverse =
 // 1 / scale (0 when scale is 0), q = clamp(round_half_away(v * inverse)).
@@ -182,7 +191,7 @@ __device__ __forceinline__ void q8_half_wave(float v, float& q, float& scale) {
   const float mx = half_wave_max(fabsf(v));
   scale = mx / 127.0f;
   const float inv = scale == 0.0f ? 0.0f : 1.0f / scale;
-  q = fminf(fmaxf(roundf(v * inv), -127.0f), 127.0f);
+  q = fminf(fmaxf(roundf(q8_product(v, inv)), -127.0f), 127.0f);
 }
 
 // One Q8 code's two sign-magnitude digits (q = 16 high + low, both carrying
@@ -285,7 +294,7 @@ __device__ __forceinline__ void residual_q8_store_n(const float (&v)[N], const b
   }
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    q[i] = fminf(fmaxf(roundf(v[i] * inv[i]), -127.0f), 127.0f);
+    q[i] = fminf(fmaxf(roundf(q8_product(v[i], inv[i])), -127.0f), 127.0f);
     r[i] = RESIDUAL ? v[i] - q[i] * s[i] : 0.0f;  // quantize_q8: no residual block
     mx[i] = fabsf(r[i]);
   }
@@ -301,7 +310,7 @@ __device__ __forceinline__ void residual_q8_store_n(const float (&v)[N], const b
     }
   }
 #pragma unroll
-  for (int i = 0; i < N; ++i) rq[i] = fminf(fmaxf(roundf(r[i] * inv[i]), -127.0f), 127.0f);
+  for (int i = 0; i < N; ++i) rq[i] = fminf(fmaxf(roundf(q8_product(r[i], inv[i])), -127.0f), 127.0f);
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     if (!live[i]) continue;  // uniform per half wave
@@ -2156,7 +2165,7 @@ __device__ __forceinline__ float wide_quantize(float (&v)[8], int sub, uint8_t* 
   uint32_t lo0 = 0, lo1 = 0, hi0 = 0, hi1 = 0;  // 48 bits of each digit
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const float q = __builtin_amdgcn_fmed3f(round_half_away(v[i] * inv), -127.0f, 127.0f);
+    const float q = __builtin_amdgcn_fmed3f(round_half_away(q8_product(v[i], inv)), -127.0f, 127.0f);
     v[i] = v[i] - q * scale;
     const uint32_t mag = __float_as_uint(fabsf(q) + 8388608.0f);  // |q| in the low bits (2^23 + |q|)
     const uint32_t sign = (__float_as_uint(q) >> 31) << 5;
@@ -2203,7 +2212,7 @@ __device__ __forceinline__ float quad_quantize(float (&v)[8], half8& code) {
   const float inv = scale == 0.0f ? 0.0f : 1.0f / scale;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const float q = __builtin_amdgcn_fmed3f(round_half_away(v[i] * inv), -127.0f, 127.0f);
+    const float q = __builtin_amdgcn_fmed3f(round_half_away(q8_product(v[i], inv)), -127.0f, 127.0f);
     v[i] = v[i] - q * scale;
     code[i] = (_Float16)q;
   }

@@ -151,7 +151,7 @@ Q8Block quantize_q8_block(const float* v, float mx) {
   for (int i = 0; i < kBlock; ++i) {
     float q = std::round(v[i] * inv);
     q = std::min(std::max(q, -127.0f), 127.0f);
-    b.values[i] = (int8_t)q;
+    b.values[i] = q == q ? (int8_t)q : 0;  // 0 x an infinite inverse: Rust's `as i8` of NaN is 0
   }
   b.scale = scale;
   return b;

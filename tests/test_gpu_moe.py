@@ -163,6 +163,36 @@ def test_exact_bf16_rows_longer_than_lds(ctx, hidden, inter):
     close(layer)
 
 
+@pytest.mark.parametrize("projection", [G.PROJECTION_RESIDUAL_Q8, G.PROJECTION_Q8], ids=["residual-q8", "q8"])
+@pytest.mark.parametrize("experts,m,inject", [(8, 1, False), (8, 3, False), (8, 5, False), (8, 5, True),
+                                              (8, 40, False), (32, 400, False), (32, 400, True), (32, 1100, False)])
+def test_blocks_whose_scale_has_no_finite_inverse(ctx, projection, experts, m, inject):
+    """Blocks of values around 1e-37 with zeros among them: the scale is below
+    2^-128, its inverse infinite, and a zero's code is 0 (0 x infinity is NaN,
+    which `as i8` makes 0). Every quantizer: the one-row, 2-4-row and tiled
+    routers, the selection kernels, and the GEMMs' epilogues; without the
+    traces too, on zero biases, so that the outputs show the codes."""
+    host = O.synthetic_layer(61, 0, experts=experts, hidden=96, intermediate=64, top_k=4)
+    host.gate_up_bias, host.down_bias = np.zeros_like(host.gate_up_bias), np.zeros_like(host.down_bias)
+    for w in (host.gate_up, host.down):
+        records = w.reshape(-1, 17)
+        records[:, 0] = 125 + np.arange(records.shape[0]) % 4
+    rng = np.random.default_rng(m)
+    x = (rng.standard_normal((m, 96)) * 1e-37).astype(np.float32)
+    x[rng.random((m, 96)) < 0.3] = 0.0
+    x[rng.random((m, 96)) < 0.1] = -0.0
+    x = synth.bf16_bits(x)
+    logits = O.bf16_round_array(rng.standard_normal((m, experts)).astype(np.float32)) if inject else None
+    want = O.moe_batch(host, x, injected_logits=logits, trace=True, projection=projection)
+    assert want["status"] == O.OK and (want["output"] != 0).any()
+    layer = gpu_layer(ctx, host, projection)
+    assert_moe_equal(layer.forward(x, injected_logits=logits), want)
+    got = layer.forward(x, injected_logits=logits, trace=True)
+    assert_moe_equal(got, want)
+    assert_traces_equal(got, want)
+    close(layer)
+
+
 def test_unknown_projection_is_rejected(ctx):
     host = O.synthetic_layer(3, 0, experts=2, hidden=64, intermediate=32, top_k=1)
     with pytest.raises(G.GossmxError) as e:
